@@ -33,7 +33,13 @@ struct Ops {
   // worth a workgroup (the MLP loss over its data points)
   static constexpr bool kGroupPso = F::id == obj::kMlp;
   using PsoEval = typename dev::GroupEvalSelect<F, 256, Gradient::Adjoint>::type;
-  static constexpr int kPsoPpb = kMfmaPso ? dev::kPsoTile : kGroupPso ? dev::kPsoGroupPpb : 256;
+  // PSO with a team of lanes per particle: the separable objectives beyond
+  // four coordinates and the binned likelihood
+  static constexpr int kPsoTeam = dev::pso_team_size<F, D>();
+  static constexpr int kPsoPpb = kMfmaPso        ? dev::kPsoTile
+                                 : kGroupPso     ? dev::kPsoGroupPpb
+                                 : kPsoTeam != 0 ? 256 / (kPsoTeam != 0 ? kPsoTeam : 1)
+                                                 : 256;
 
   static hipError_t pso(const dev::PsoArgs& a, int nb, hipStream_t s)
   {
@@ -44,6 +50,8 @@ struct Ops {
     else if constexpr (kGroupPso)
       dev::pso_group_kernel<F, D, 256, kPsoPpb, PsoEval, dev::BuiltinProvider>
         <<<nb, 256, 0, s>>>(a, {});
+    else if constexpr (kPsoTeam != 0)
+      dev::pso_team_kernel<F, D, kPsoTeam, dev::BuiltinProvider><<<nb, 256, 0, s>>>(a, {});
     else
       dev::pso_lane_kernel<F, D, dev::BuiltinProvider><<<nb, 256, 0, s>>>(a, {});
     return hipGetLastError();
@@ -54,7 +62,7 @@ struct Ops {
   {
     if (fault_take_launch())
       return hipErrorLaunchFailure;
-    dev::pso_final_kernel<256, kPsoPpb, D><<<n_probs, 256, 0, s>>>(a);
+    dev::pso_final_kernel<256, D><<<n_probs, 256, 0, s>>>(a);
     return hipGetLastError();
   }
 
@@ -280,6 +288,7 @@ struct Ops {
       o.objective = F::id;
       o.dim = D;
       o.pso_ppb = kPsoPpb;
+      o.pso_team = kPsoTeam != 0;
       o.pso = &pso;
       o.pso_final = &pso_final;
       o.thread_ok = kThreadOk;

@@ -19,6 +19,7 @@ struct ClassOps {
   int objective = 0;
   int dim = 0;
   int pso_ppb = 256; // particles per PSO workgroup
+  bool pso_team = false; // a workgroup may take pso_ppb x 2^k particles (team form)
   hipError_t (*pso)(const dev::PsoArgs&, int nblocks, hipStream_t) = nullptr;
   hipError_t (*pso_final)(const dev::PsoArgs&, int n_probs, hipStream_t) = nullptr;
   bool thread_ok = false;
@@ -44,6 +45,19 @@ struct ClassOps {
   hipError_t (*eval)(const dev::ProblemDesc&, const double* x, int64_t n, double* f,
                      double* g, int gradient, hipStream_t) = nullptr;
 };
+
+// Particles per PSO workgroup for problems of up to n_starts starts: the team
+// form takes more passes per workgroup once a problem would have more than
+// kPsoMaxBlocks workgroups.
+inline int
+pso_ppb_for(const ClassOps* ops, int64_t n_starts)
+{
+  int ppb = ops->pso_ppb;
+  if (ops->pso_team)
+    while ((n_starts + ppb - 1) / ppb > dev::kPsoMaxBlocks && ppb < (1 << 24))
+      ppb *= 2;
+  return ppb;
+}
 
 // Registry (one function per instantiation unit).
 const ClassOps* find_class(int objective, int dim);

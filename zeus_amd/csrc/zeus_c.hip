@@ -365,6 +365,7 @@ struct ClassPlan {
   std::vector<int> probs; // indices into the caller's problem array
   int64_t total = 0;
   int pso_blocks = 0;
+  int ppb = 256; // particles per PSO workgroup
   int max_pso_iter = -1;
   TuneVal cfg{};
   std::vector<TuneVal> cands; // > 1 entry: time them and keep the fastest
@@ -453,7 +454,7 @@ pso_args(const ClassPlan& c, Control* ctl)
                  c.part_val, c.part_idx,
                  c.part_x,   c.gstate,
                  c.d_block_problem, c.xw,
-                 c.total * c.ops->dim, c.keep_rng};
+                 c.total * c.ops->dim, c.keep_rng, c.ppb};
 }
 
 // Objective preparation and PSO iterations t0 .. max_pso_iter of a class.
@@ -645,8 +646,11 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
   for (auto& c : classes) {
     c.ctl0 = ctl_total;
     ctl_total += int(c.probs.size());
-    int64_t s0 = 0;
+    int64_t s0 = 0, n_max = 0;
     int b0 = 0;
+    for (int pi : c.probs)
+      n_max = std::max(n_max, probs[pi].n_starts);
+    c.ppb = rt::pso_ppb_for(c.ops, n_max);
     for (int pi : c.probs) {
       const zeus_problem& p = probs[pi];
       ProblemDesc d{};
@@ -672,7 +676,7 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
       d.traj = traj_of(p);
       c.traced = c.traced || d.traj.fval != nullptr;
       c.desc.push_back(d);
-      const int nb = int((p.n_starts + c.ops->pso_ppb - 1) / c.ops->pso_ppb);
+      const int nb = int((p.n_starts + c.ppb - 1) / c.ppb);
       for (int b = 0; b < nb; ++b)
         c.block_problem.push_back(int32_t(c.desc.size() - 1));
       b0 += nb;
@@ -1242,7 +1246,8 @@ pso_phase(const zeus_problem* prob, int t0, int t1, double* X, double* V, double
   d.n_params = prob->n_params;
   c.desc.push_back(d);
   c.xorwow = d.prng == ZEUS_PRNG_XORWOW && t1 > 0 && xw == nullptr;
-  c.pso_blocks = int((prob->n_starts + c.ops->pso_ppb - 1) / c.ops->pso_ppb);
+  c.ppb = rt::pso_ppb_for(c.ops, prob->n_starts);
+  c.pso_blocks = int((prob->n_starts + c.ppb - 1) / c.ppb);
   c.block_problem.assign(c.pso_blocks, 0);
   c.total = prob->n_starts;
   c.max_pso_iter = t1;
@@ -1350,26 +1355,44 @@ pso_run_noalloc(const zeus_problem* prob, double* pbx, double* pbv, double* gbx_
   const ClassOps* ops = rt::find_class(prob->objective, prob->dim);
   const int D = prob->dim;
   const int64_t n = prob->n_starts;
-  const int nb = int((n + ops->pso_ppb - 1) / ops->pso_ppb);
   const int T = prob->pso_iter;
   const bool gauss = ops->objective == obj::kGaussian;
   const bool xorwow = prob->prng == ZEUS_PRNG_XORWOW && T > 0;
 
-  Carver cv{static_cast<char*>(base)};
-  ProblemDesc* d_desc = cv.take<ProblemDesc>(1);
-  int32_t* d_bp = cv.take<int32_t>(size_t(nb));
-  double* X = cv.take<double>(size_t(n) * D);
-  double* V = cv.take<double>(size_t(n) * D);
-  double* gbx = gbx_out ? gbx_out : cv.take<double>(size_t(D));
-  double* part_val = cv.take<double>(2 * size_t(nb));
-  int64_t* part_idx = cv.take<int64_t>(2 * size_t(nb));
-  double* part_x = cv.take<double>(2 * size_t(nb) * D);
-  double* gstate = cv.take<double>(2 * size_t(D + 1));
-  double* aux = gauss ? cv.take<double>(size_t(dev::gaussian_aux_doubles(D))) : nullptr;
-  uint32_t* xw = xorwow ? cv.take<uint32_t>(6 * size_t(n) * D) : nullptr;
-  Control* ctl = cv.take<Control>(1);
-  if (cv.off > kScratchBytes)
-    return ZEUS_E_SCRATCH;
+  ProblemDesc* d_desc = nullptr;
+  int32_t* d_bp = nullptr;
+  double *X = nullptr, *V = nullptr, *gbx = nullptr, *part_val = nullptr, *part_x = nullptr;
+  double *gstate = nullptr, *aux = nullptr;
+  int64_t* part_idx = nullptr;
+  uint32_t* xw = nullptr;
+  Control* ctl = nullptr;
+  int nb = 0;
+  auto carve = [&](int ppb) {
+    Carver cv{static_cast<char*>(base)};
+    nb = int((n + ppb - 1) / ppb);
+    d_desc = cv.take<ProblemDesc>(1);
+    d_bp = cv.take<int32_t>(size_t(nb));
+    X = cv.take<double>(size_t(n) * D);
+    V = cv.take<double>(size_t(n) * D);
+    gbx = gbx_out ? gbx_out : cv.take<double>(size_t(D));
+    part_val = cv.take<double>(2 * size_t(nb));
+    part_idx = cv.take<int64_t>(2 * size_t(nb));
+    part_x = cv.take<double>(2 * size_t(nb) * D);
+    gstate = cv.take<double>(2 * size_t(D + 1));
+    aux = gauss ? cv.take<double>(size_t(dev::gaussian_aux_doubles(D))) : nullptr;
+    xw = xorwow ? cv.take<uint32_t>(6 * size_t(n) * D) : nullptr;
+    ctl = cv.take<Control>(1);
+    return cv.off <= kScratchBytes;
+  };
+  // The team form's partials grow with the workgroup count: where they would
+  // not fit, a workgroup takes more particles (the swarm does not depend on
+  // it), down to the 256 that the lane form has.
+  int ppb = rt::pso_ppb_for(ops, n);
+  while (!carve(ppb)) {
+    if (!ops->pso_team || ppb >= 256)
+      return ZEUS_E_SCRATCH;
+    ppb *= 2;
+  }
 
   ProblemDesc d{};
   d.objective = prob->objective;
@@ -1397,7 +1420,7 @@ pso_run_noalloc(const zeus_problem* prob, double* pbx, double* pbv, double* gbx_
     e = hipGetLastError();
   }
   PsoArgs pa{d_desc, 1,    0,        nb,       ctl,    X,    V,         pbx, pbv,
-             gbx,    part_val, part_idx, part_x, gstate, d_bp, xw, n * D, 0};
+             gbx,    part_val, part_idx, part_x, gstate, d_bp, xw, n * D, 0,   ppb};
   for (int it = 0; e == hipSuccess && it <= T; ++it) {
     pa.iter = it;
     e = ops->pso(pa, nb, st);
