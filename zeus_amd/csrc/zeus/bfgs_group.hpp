@@ -230,28 +230,64 @@ struct GroupEvalSeparable {
 };
 
 // ---------------------------------------------------------------------------
-// Poisson NLL: bins spread over the lanes.
+// Poisson NLL: bins spread over the lanes; the first kKeep bins of a lane are
+// held in registers from problem to problem.  The dual gradient makes its four
+// forward passes bin by bin on the bin's lane.
 template <int NT, Gradient G>
 struct GroupEvalLogLik {
   using F = obj::LogLikelihood;
+  static constexpr int kKeep = 2;
   GroupScratch sc;
-  ZEUS_D void bind(const ProblemDesc&) {}
+  F::Bin kept[kKeep];
+
+  ZEUS_D void bind(const ProblemDesc& P)
+  {
+    const F f{P.params, int(P.n_params / 3), P.aux};
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      const int i = int(threadIdx.x) + j * NT;
+      if (f.T != nullptr && i < f.n)
+        kept[j] = f.bin(i);
+    }
+  }
+  // fn(bin) over this lane's bins in order (f.T != nullptr)
+  template <class Fn>
+  ZEUS_D ZEUS_FI void each_bin(const F& f, Fn&& fn)
+  {
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j)
+      if (int(threadIdx.x) + j * NT < f.n)
+        fn(kept[j]);
+    for (int i = threadIdx.x + kKeep * NT; i < f.n; i += NT)
+      fn(f.bin(i));
+  }
   ZEUS_D double value(const F& f, const double* th, Block<NT>& blk)
   {
-    const double t0 = th[0], t1 = th[1], t2 = th[2], t3 = th[3];
-    const double tt[4] = {t0, t1, t2, t3};
     double t = 0.0;
-    for (int i = threadIdx.x; i < f.n; i += NT)
-      t += f.bin_value(tt, i);
+    if (f.T != nullptr) {
+      const F::Theta h(th);
+      each_bin(f, [&](const F::Bin& v) { t += F::bin_term(h, v); });
+    } else {
+      for (int i = threadIdx.x; i < f.n; i += NT)
+        t -= f.template bin_log_p<double>(obj::PtrView{th}, i);
+    }
     return blk.sum1(t);
   }
   ZEUS_D void gradient(const F& f, const double* th, double* g, bool, Block<NT>& blk)
   {
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
     if constexpr (G == Gradient::Dual) {
-      group_dual_gradient<F, 4, NT>(f, th, g);
+#pragma unroll 1
+      for (int i = threadIdx.x; i < f.n; i += NT)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          v[k] -= f.template bin_log_p<dual::DualNumber>(obj::SeededView{th, k}, i).dual;
+    } else if (f.T != nullptr) {
+      const F::Theta h(th);
+      const double ra = 1.0 / h.a;
+      each_bin(f, [&](const F::Bin& b) { (void)F::bin_gradient(h, ra, b, v); });
     } else {
       const double a = th[0], b = th[1], c = th[2], d = th[3];
-      double v[4] = {0.0, 0.0, 0.0, 0.0};
       for (int i = threadIdx.x; i < f.n; i += NT) {
         const double x = f.P[i];
         const double k = f.P[f.n + i];
@@ -266,10 +302,10 @@ struct GroupEvalLogLik {
         v[2] -= wm * lx;
         v[3] -= wm * (lx * lx);
       }
-      blk.template sum<4>(v);
-      if (threadIdx.x < 4)
-        g[threadIdx.x] = v[threadIdx.x];
     }
+    blk.template sum<4>(v);
+    if (threadIdx.x < 4)
+      g[threadIdx.x] = v[threadIdx.x];
   }
 };
 

@@ -18,6 +18,7 @@
 //   Mlp           x (P), y (P)                       1-16-16-1 tanh, MSE
 #pragma once
 
+#include "binned.hpp"
 #include "dual.hpp"
 #include "traits.hpp"
 
@@ -258,68 +259,127 @@ struct Gaussian {
 // mu_i = a (1 - x_i)^b / x_i^(c + d ln x_i);  f = -sum_i [k_i ln mu_i - mu_i
 // - lgamma(k_i + 1)].  The lgamma(k+1) constants come precomputed in the
 // parameter block (they do not depend on the parameters being fitted).
+// With the table of the bins' logarithms (binned.hpp, prepared once per call)
+// a double evaluation is one exponential per bin; without it, and in dual
+// numbers, the power functions.
 struct LogLikelihood {
   static constexpr std::size_t arity = 4;
   static constexpr int id = kLogLikelihood;
   const double* P = nullptr; // [x (n) | k (n) | lgamma(k+1) (n)]
   int n = 0;
+  const double* T = nullptr; // [ln x | rest | ln(1 - x) | rest], n each, or null
 
-  template <class T, class X>
-  ZEUS_HD T eval(const X& th) const
+  // the parameters and what every bin needs of them
+  struct Theta {
+    double a, b, c, d, la;
+    bool a_plain;
+    ZEUS_HD explicit Theta(const double* th)
+      : a(th[0]), b(th[1]), c(th[2]), d(th[3]), la(::log(th[0])),
+        a_plain(th[0] >= 1e-30 && th[0] <= 1e30)
+    {
+    }
+  };
+  // one bin: center, count, lgamma(count + 1) and the logarithms
+  struct Bin {
+    double x, k, lgk;
+    dev::BinLogs t;
+  };
+  ZEUS_HD Bin bin(int i) const
+  {
+    return {P[i], P[n + i], P[2 * n + i], {T[i], T[n + i], T[2 * n + i], T[3 * n + i]}};
+  }
+  ZEUS_HD static double bin_term(const Theta& h, const Bin& v)
+  {
+    const dev::BinMean m = dev::bin_mean(h.a, h.b, h.c, h.d, h.la, h.a_plain, v.x, v.t);
+    return -(v.k * m.log_mean - m.mean - v.lgk);
+  }
+  // adds the bin's gradient terms and returns its value; ra = 1 / a
+  ZEUS_HD static double bin_gradient(const Theta& h, double ra, const Bin& v, double (&g)[4])
+  {
+    const dev::BinMean m = dev::bin_mean(h.a, h.b, h.c, h.d, h.la, h.a_plain, v.x, v.t);
+    double wm, ga; // mean x d nll / d mean, and d nll / d a
+    if (m.plain) {
+      wm = m.mean - v.k;
+      ga = wm * ra;
+    } else {
+      const double w = 1.0 - v.k / m.mean;
+      wm = w * m.mean;
+      ga = w * m.ratio;
+    }
+    g[0] += ga;
+    // ln(1 - x) is NaN in the table where the power functions are used
+    g[1] += wm * (v.t.l1 == v.t.l1 ? v.t.l1 : ::log(1.0 - v.x));
+    g[2] -= wm * v.t.lx;
+    g[3] -= wm * (v.t.lx * v.t.lx);
+    return -(v.k * m.log_mean - m.mean - v.lgk);
+  }
+
+  // one bin's contribution in T = double (power functions) or dual numbers
+  template <class T_, class X>
+  ZEUS_HD T_ bin_log_p(const X& th, int i) const
   {
     using ::log;
     using ::pow;
     using dual::log;
     using dual::pow;
-    const T a = th[0], b = th[1], c = th[2], d = th[3];
-    T nll = T(0.0);
-    for (int i = 0; i < n; ++i) {
-      const T x = T(P[i]);
-      const T k = T(P[n + i]);
-      const T mean = a * pow(T(1.0) - x, b) / pow(x, c + d * log(x));
-      const T log_p = k * log(mean) - mean - T(P[2 * n + i]);
-      nll -= log_p;
+    const T_ a = th[0], b = th[1], c = th[2], d = th[3];
+    const T_ x = T_(P[i]);
+    const T_ k = T_(P[n + i]);
+    const T_ mean = a * pow(T_(1.0) - x, b) / pow(x, c + d * log(x));
+    return k * log(mean) - mean - T_(P[2 * n + i]);
+  }
+  template <class T_, class X>
+  ZEUS_HD T_ eval(const X& th) const
+  {
+    T_ nll = T_(0.0);
+    if constexpr (kIsDouble<T_>) {
+      if (T != nullptr) {
+        const double v[4] = {th[0], th[1], th[2], th[3]};
+        const Theta h(v);
+        for (int i = 0; i < n; ++i)
+          nll += bin_term(h, bin(i));
+        return nll;
+      }
     }
+    for (int i = 0; i < n; ++i)
+      nll -= bin_log_p<T_>(th, i);
     return nll;
   }
-  template <class T>
-  ZEUS_HD T operator()(const std::array<T, 4>& x) const
+  template <class T_>
+  ZEUS_HD T_ operator()(const std::array<T_, 4>& x) const
   {
-    return eval<T>(ArrayView<T, 4>{x});
+    return eval<T_>(ArrayView<T_, 4>{x});
   }
   ZEUS_HD double value_and_gradient(const double* th, double* g) const
   {
-    const double a = th[0], b = th[1], c = th[2], d = th[3];
-    double nll = 0.0, ga = 0.0, gb = 0.0, gc = 0.0, gd = 0.0;
-    for (int i = 0; i < n; ++i) {
-      const double x = P[i];
-      const double k = P[n + i];
-      const double lx = ::log(x);
-      const double pw = ::pow(1.0 - x, b);
-      const double qw = ::pow(x, c + d * lx);
-      const double mean = a * pw / qw;
-      const double log_p = k * ::log(mean) - mean - P[2 * n + i];
-      nll -= log_p;
-      const double w = 1.0 - k / mean; // d nll / d mean
-      const double wm = w * mean;
-      ga += w * (pw / qw);
-      gb += wm * ::log(1.0 - x);
-      gc -= wm * lx;
-      gd -= wm * (lx * lx);
+    double nll = 0.0, v[4] = {0.0, 0.0, 0.0, 0.0};
+    if (T != nullptr) {
+      const Theta h(th);
+      const double ra = 1.0 / h.a;
+      for (int i = 0; i < n; ++i)
+        nll += bin_gradient(h, ra, bin(i), v);
+    } else {
+      const double a = th[0], b = th[1], c = th[2], d = th[3];
+      for (int i = 0; i < n; ++i) {
+        const double x = P[i];
+        const double k = P[n + i];
+        const double lx = ::log(x);
+        const double pw = ::pow(1.0 - x, b);
+        const double qw = ::pow(x, c + d * lx);
+        const double mean = a * pw / qw;
+        const double log_p = k * ::log(mean) - mean - P[2 * n + i];
+        nll -= log_p;
+        const double w = 1.0 - k / mean; // d nll / d mean
+        const double wm = w * mean;
+        v[0] += w * (pw / qw);
+        v[1] += wm * ::log(1.0 - x);
+        v[2] -= wm * lx;
+        v[3] -= wm * (lx * lx);
+      }
     }
-    g[0] = ga;
-    g[1] = gb;
-    g[2] = gc;
-    g[3] = gd;
+    for (int i = 0; i < 4; ++i)
+      g[i] = v[i];
     return nll;
-  }
-  // One data bin's contribution (used by the cooperative evaluator).
-  ZEUS_HD double bin_value(const double* th, int i) const
-  {
-    const double x = P[i];
-    const double k = P[n + i];
-    const double mean = th[0] * ::pow(1.0 - x, th[1]) / ::pow(x, th[2] + th[3] * ::log(x));
-    return -(k * ::log(mean) - mean - P[2 * n + i]);
   }
 };
 

@@ -128,6 +128,53 @@ gaussian_aux_doubles(int D)
   return int64_t(D) * D + (int64_t(MB) * KB + nu) * 64;
 }
 
+// Bins of a likelihood whose logarithms are tabulated; beyond, the bins are
+// evaluated with the power functions (the single-problem entry points keep
+// their table in a fixed device array of this size).
+constexpr int64_t kMaxTableBins = 16384;
+inline int64_t
+loglik_aux_doubles(int64_t n_params)
+{
+  return n_params / 3 <= kMaxTableBins ? kBinLogs * (n_params / 3) : 0;
+}
+
+// The table of a problem's bins' logarithms (binned.hpp), one logarithm per
+// thread.
+ZEUS_D inline void
+bin_table(const ProblemDesc& P)
+{
+  const int n = int(P.n_params / 3);
+  if (P.aux == nullptr)
+    return;
+  double* T = const_cast<double*>(P.aux);
+  for (int e = threadIdx.x; e < 2 * n; e += blockDim.x) {
+    const int i = e < n ? e : e - n;
+    const DD l = e < n ? bin_log_x(P.params[i]) : bin_log_1mx(P.params[i]);
+    T[(e < n ? 0 : 2 * n) + i] = l.hi;
+    T[(e < n ? n : 3 * n) + i] = l.lo;
+  }
+}
+// one workgroup per problem
+static __global__ void
+bin_table_kernel(const ProblemDesc* desc)
+{
+  bin_table(desc[blockIdx.x]);
+}
+// init_controls_kernel and bin_table_kernel in one launch, for a call whose
+// first class is the likelihood (the grid covers its np problems).
+static __global__ void
+init_bin_table_kernel(Control* c, int n, double* gbx, int64_t n_gbx, const ProblemDesc* desc,
+                      int np)
+{
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n)
+    reset_control(c + i);
+  for (int64_t kk = i; kk < n_gbx; kk += int64_t(gridDim.x) * blockDim.x)
+    gbx[kk] = 0.0;
+  if (int(blockIdx.x) < np)
+    bin_table(desc[blockIdx.x]);
+}
+
 // One workgroup per problem: deterministic argmin of the start values (the
 // reference's launchReduction, bfgs_common.cuh:280-319, with NaN skipped
 // and ties to the lowest index) plus the status counts of
@@ -257,6 +304,7 @@ struct BuiltinProvider {
     } else if constexpr (F::id == obj::kLogLikelihood) {
       f.P = P.params;
       f.n = int(P.n_params / 3);
+      f.T = P.aux;
     } else if constexpr (F::id == obj::kMlp) {
       f.P = P.params;
       f.m = int(P.n_params / 2);

@@ -381,7 +381,8 @@ struct ClassPlan {
   double* part_x = nullptr;    // [2][pso_blocks][D]
   double* gstate = nullptr;    // per problem [2][1 + D]
   StartOut out{};
-  double* aux = nullptr; // Gaussian Cs, one D x D block per problem
+  double* aux = nullptr; // prepared objective data, one block per problem
+  int64_t aux_total = 0; // its doubles
   double* h_slab = nullptr;
   int ctl0 = 0;          // first control block of the class
   bool traced = false;   // some problem records a trajectory
@@ -394,6 +395,30 @@ struct ClassPlan {
   std::vector<ProblemDesc> desc;
   std::vector<int32_t> block_problem;
 };
+
+// Doubles of a problem's prepared objective data: the Gaussian's symmetric
+// matrix and its MFMA fragments, the likelihood's table of logarithms.
+int64_t
+aux_doubles(int objective, int dim, int64_t n_params)
+{
+  return objective == obj::kGaussian        ? dev::gaussian_aux_doubles(dim)
+         : objective == obj::kLogLikelihood ? dev::loglik_aux_doubles(n_params)
+                                            : 0;
+}
+
+// Points the descriptors at their blocks of the class's prepared data.
+void
+bind_aux(ClassPlan& c)
+{
+  int64_t o = 0;
+  for (auto& d : c.desc) {
+    const int64_t n = aux_doubles(d.objective, d.dim, d.n_params);
+    d.aux = n > 0 ? c.aux + o : nullptr;
+    if (d.objective == obj::kGaussian)
+      d.aux_frag = d.aux + int64_t(d.dim) * d.dim;
+    o += n;
+  }
+}
 
 // Host-written inputs of a class (uploaded in one copy with the others).
 void
@@ -426,8 +451,7 @@ carve_class(Carver& cv, ClassPlan& c)
   c.out.fval = cv.take<double>(n);
   c.out.gnorm = cv.take<double>(n);
   c.out.x = cv.take<double>(n * D);
-  c.aux = cv.take<double>(c.ops->objective == obj::kGaussian ? np * dev::gaussian_aux_doubles(D)
-                                                              : 1);
+  c.aux = cv.take<double>(size_t(std::max<int64_t>(c.aux_total, 1)));
   c.h_slab = cv.take<double>(size_t(std::max<int64_t>(c.slab, 1)));
   if (c.xorwow)
     c.xw = cv.take<uint32_t>(6 * n * D);
@@ -472,6 +496,11 @@ launch_class(ClassPlan& c, Control* ctl_all, int gradient, hipStream_t st, int t
       dev::symmetrize_kernel<<<int((na + 255) / 256), 256, 0, st>>>(c.d_desc, k, cs,
                                                                     cs + int64_t(D) * D, D);
     }
+    if ((e = hipGetLastError()) != hipSuccess)
+      return e;
+  }
+  if (c.ops->objective == obj::kLogLikelihood && !c.prepared && c.aux_total > 0) {
+    dev::bin_table_kernel<<<np, 256, 0, st>>>(c.d_desc);
     if ((e = hipGetLastError()) != hipSuccess)
       return e;
   }
@@ -675,6 +704,7 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
       c.xorwow = c.xorwow || (d.prng == ZEUS_PRNG_XORWOW && d.pso_iter > 0);
       d.traj = traj_of(p);
       c.traced = c.traced || d.traj.fval != nullptr;
+      c.aux_total += aux_doubles(d.objective, d.dim, d.n_params);
       c.desc.push_back(d);
       const int nb = int((p.n_starts + c.ppb - 1) / c.ppb);
       for (int b = 0; b < nb; ++b)
@@ -757,11 +787,9 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
     for (auto& d : c.desc) {
       if (d.x0 == nullptr && d.pso_iter >= 0)
         d.x0 = c.pbx + d.start0 * d.dim;
-      if (c.ops->objective == obj::kGaussian) {
-        d.aux = c.aux + (&d - c.desc.data()) * dev::gaussian_aux_doubles(d.dim);
-        d.aux_frag = d.aux + int64_t(d.dim) * d.dim;
-      }
     }
+  for (auto& c : classes)
+    bind_aux(c);
   // best-x offsets per control block (class order)
   std::vector<int64_t> bxo(ctl_total);
   std::vector<int64_t> bx_user(n_probs);
@@ -850,6 +878,11 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
         const int64_t n = std::max<int64_t>(ctl_total, na);
         dev::init_symmetrize_kernel<<<int((n + 255) / 256), 256, 0, st>>>(
           d_ctl, ctl_total, c.gbx, ng, c.d_desc, 0, c.aux, c.aux + int64_t(D) * D, D);
+      } else if (i == 0 && c.ops->objective == obj::kLogLikelihood) {
+        const int np = int(c.probs.size());
+        const int g = std::max((ctl_total + 255) / 256, np);
+        dev::init_bin_table_kernel<<<g, 256, 0, st>>>(d_ctl, ctl_total, c.gbx, ng, c.d_desc, np);
+        c.prepared = true;
       } else if (i == 0)
         dev::init_controls_kernel<<<(ctl_total + 255) / 256, 256, 0, st>>>(d_ctl, ctl_total,
                                                                            c.gbx, ng);
@@ -961,6 +994,7 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
       key.push_back(uint64_t(c.probs.size()));
       key.push_back(uint64_t(c.cfg.form) << 32 | uint32_t(c.cfg.threads));
       key.push_back(uint64_t(c.xorwow));
+      key.push_back(uint64_t(c.aux_total));
       key.push_back(uint64_t(c.metrics));
     }
     key.push_back(uint64_t(concurrent));
@@ -1245,6 +1279,7 @@ pso_phase(const zeus_problem* prob, int t0, int t1, double* X, double* V, double
   d.params = prob->params;
   d.n_params = prob->n_params;
   c.desc.push_back(d);
+  c.aux_total = aux_doubles(d.objective, d.dim, d.n_params);
   c.xorwow = d.prng == ZEUS_PRNG_XORWOW && t1 > 0 && xw == nullptr;
   c.ppb = rt::pso_ppb_for(c.ops, prob->n_starts);
   c.pso_blocks = int((prob->n_starts + c.ppb - 1) / c.ppb);
@@ -1278,10 +1313,7 @@ pso_phase(const zeus_problem* prob, int t0, int t1, double* X, double* V, double
   c.pbv = pbv;
   if (gbx)
     c.gbx = gbx;
-  if (c.ops->objective == obj::kGaussian) {
-    c.desc[0].aux = c.aux;
-    c.desc[0].aux_frag = c.aux + int64_t(prob->dim) * prob->dim;
-  }
+  bind_aux(c);
   hipError_t e = hipMemcpyAsync(c.d_desc, c.desc.data(), sizeof(ProblemDesc),
                                 hipMemcpyHostToDevice, st);
   if (e == hipSuccess)
@@ -1313,23 +1345,32 @@ pso_phase(const zeus_problem* prob, int t0, int t1, double* X, double* V, double
 constexpr size_t kScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+// The likelihood's table of logarithms of the entry points that allocate
+// nothing (the allocation-free PSO and zeus_eval), beside the scratch array so
+// that it takes nothing from it.
+static __device__ double bin_table_mem[dev::kBinLogs * dev::kMaxTableBins];
+
 constexpr int kMaxDevices = 64;
 void* g_scratch_ptr[kMaxDevices] = {};
+void* g_table_ptr[kMaxDevices] = {};
 
-// Address of the current device's scratch array (resolved once per device).
+// Addresses of the current device's fixed arrays (resolved once per device).
 zeus_status_t
-scratch_base(void** out)
+fixed_arrays(void** scratch_out, double** table_out)
 {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
     return ZEUS_E_NODEVICE;
   if (!g_scratch_ptr[dev]) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p)
+    void *p = nullptr, *t = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p ||
+        hipGetSymbolAddress(&t, HIP_SYMBOL(bin_table_mem)) != hipSuccess || !t)
       return ZEUS_E_LAUNCH;
     g_scratch_ptr[dev] = p;
+    g_table_ptr[dev] = t;
   }
-  *out = g_scratch_ptr[dev];
+  *scratch_out = g_scratch_ptr[dev];
+  *table_out = static_cast<double*>(g_table_ptr[dev]);
   return ZEUS_OK;
 }
 
@@ -1345,12 +1386,19 @@ noalloc_setup_kernel(ProblemDesc d, ProblemDesc* out, int32_t* block_problem, in
     block_problem[i] = 0;
 }
 
+// bin_table_kernel of a descriptor passed by value.
+__global__ void
+bin_table_kernel(ProblemDesc d)
+{
+  dev::bin_table(d);
+}
+
 // zeus_pso_run on the scratch array: the same kernels in the same order on
 // the same inputs, with every buffer beyond the caller's outputs carved from
 // `base` (kScratchBytes) instead of the library's arena.
 zeus_status_t
 pso_run_noalloc(const zeus_problem* prob, double* pbx, double* pbv, double* gbx_out,
-                double* gbv, void* base, hipStream_t st)
+                double* gbv, void* base, double* table, hipStream_t st)
 {
   const ClassOps* ops = rt::find_class(prob->objective, prob->dim);
   const int D = prob->dim;
@@ -1410,6 +1458,10 @@ pso_run_noalloc(const zeus_problem* prob, double* pbx, double* pbv, double* gbx_
     d.aux = aux;
     d.aux_frag = aux + int64_t(D) * D;
   }
+  const bool table_used =
+    ops->objective == obj::kLogLikelihood && dev::loglik_aux_doubles(d.n_params) > 0;
+  if (table_used)
+    d.aux = table;
   noalloc_setup_kernel<<<(std::max(nb, 1) + 255) / 256, 256, 0, st>>>(d, d_desc, d_bp, nb);
   dev::init_controls_kernel<<<1, 256, 0, st>>>(ctl, 1, gbx, D);
   hipError_t e = hipGetLastError();
@@ -1417,6 +1469,10 @@ pso_run_noalloc(const zeus_problem* prob, double* pbx, double* pbv, double* gbx_
     const int64_t na = dev::gaussian_aux_doubles(D);
     dev::symmetrize_kernel<<<int((na + 255) / 256), 256, 0, st>>>(d_desc, 0, aux,
                                                                   aux + int64_t(D) * D, D);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && table_used) {
+    dev::bin_table_kernel<<<1, 256, 0, st>>>(d_desc);
     e = hipGetLastError();
   }
   PsoArgs pa{d_desc, 1,    0,        nb,       ctl,    X,    V,         pbx, pbv,
@@ -1454,10 +1510,11 @@ zeus_pso_run_noalloc(const zeus_problem* prob, double* pbest_x, double* pbest_va
   if ((rc = ensure_device()) != ZEUS_OK)
     return rc;
   void* base = nullptr;
-  if ((rc = scratch_base(&base)) != ZEUS_OK)
+  double* table = nullptr;
+  if ((rc = fixed_arrays(&base, &table)) != ZEUS_OK)
     return rc;
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : g_ds.stream;
-  return pso_run_noalloc(prob, pbest_x, pbest_val, gbest_x, gbest_val, base, st);
+  return pso_run_noalloc(prob, pbest_x, pbest_val, gbest_x, gbest_val, base, table, st);
 }
 
 zeus_status_t
@@ -1562,6 +1619,15 @@ zeus_eval(const zeus_problem* prob, const double* x, int64_t n, double* f, doubl
   d.params = prob->params;
   d.n_params = prob->n_params;
   const ClassOps* ops = rt::find_class(prob->objective, prob->dim);
+  if (n > 0 && ops->objective == obj::kLogLikelihood &&
+      dev::loglik_aux_doubles(d.n_params) > 0) {
+    void* base = nullptr;
+    double* table = nullptr;
+    if ((rc = fixed_arrays(&base, &table)) != ZEUS_OK)
+      return rc;
+    d.aux = table;
+    bin_table_kernel<<<1, 256, 0, st>>>(d);
+  }
   hipError_t e = ops->eval(d, x, n, f, grad, gradient, st);
   const hipError_t e2 = hipStreamSynchronize(st);
   return to_status(e != hipSuccess ? e : e2);
