@@ -230,82 +230,101 @@ struct GroupEvalSeparable {
 };
 
 // ---------------------------------------------------------------------------
-// Poisson NLL: bins spread over the lanes; the first kKeep bins of a lane are
-// held in registers from problem to problem.  The dual gradient makes its four
-// forward passes bin by bin on the bin's lane.
+// Poisson NLL: bins spread over the lanes.  The first kKeep bins stay in LDS
+// from problem to problem, and their means at the last value, from which the
+// gradient there follows without evaluating the powers again; every lane reads
+// back only what it wrote.  The dual gradient makes its four forward passes
+// bin by bin on the bin's lane and adds them in bin order.
 template <int NT, Gradient G>
 struct GroupEvalLogLik {
   using F = obj::LogLikelihood;
-  static constexpr int kKeep = 2;
+  static constexpr int kKeep = 128;
+  static constexpr int kFields = 5; // x, k, lgamma(k + 1), ln x, ln(1 - x)
+  struct Lds {
+    double bin[kFields][kKeep];
+    double mean[kKeep], ratio[kKeep];
+    double dual[G == Gradient::Dual ? 4 : 1][G == Gradient::Dual ? NT : 1];
+  };
   GroupScratch sc;
-  F::Bin kept[kKeep];
+  Lds* L;
 
   ZEUS_D void bind(const ProblemDesc& P)
   {
+    __shared__ Lds lds;
+    L = &lds;
     const F f{P.params, int(P.n_params / 3), P.aux};
+    for (int i = threadIdx.x; i < f.n && i < kKeep; i += NT) {
+      const F::Bin b = f.bin(i);
+      const double v[kFields] = {b.x, b.k, b.lgk, b.t.lx, b.t.l1};
 #pragma unroll
-    for (int j = 0; j < kKeep; ++j) {
-      const int i = int(threadIdx.x) + j * NT;
-      if (f.T != nullptr && i < f.n)
-        kept[j] = f.bin(i);
+      for (int e = 0; e < kFields; ++e)
+        L->bin[e][i] = v[e];
     }
   }
-  // fn(bin) over this lane's bins in order (f.T != nullptr)
-  template <class Fn>
-  ZEUS_D ZEUS_FI void each_bin(const F& f, Fn&& fn)
+  ZEUS_D ZEUS_FI F::Bin bin(const F& f, int i) const
   {
-#pragma unroll
-    for (int j = 0; j < kKeep; ++j)
-      if (int(threadIdx.x) + j * NT < f.n)
-        fn(kept[j]);
-    for (int i = threadIdx.x + kKeep * NT; i < f.n; i += NT)
-      fn(f.bin(i));
+    if (i >= kKeep)
+      return f.bin(i);
+    return {L->bin[0][i], L->bin[1][i], L->bin[2][i], {L->bin[3][i], 0.0, L->bin[4][i], 0.0}};
   }
   ZEUS_D double value(const F& f, const double* th, Block<NT>& blk)
   {
+    const double a = th[0], b = th[1], c = th[2], d = th[3];
     double t = 0.0;
-    if (f.T != nullptr) {
-      const F::Theta h(th);
-      each_bin(f, [&](const F::Bin& v) { t += F::bin_term(h, v); });
-    } else {
-      for (int i = threadIdx.x; i < f.n; i += NT)
-        t -= f.template bin_log_p<double>(obj::PtrView{th}, i);
+#pragma unroll 1
+    for (int i = threadIdx.x; i < f.n; i += NT) {
+      const F::Bin e = bin(f, i);
+      const BinPow m = bin_pow(a, b, c, d, e.x, e.t);
+      if (i < kKeep) {
+        L->mean[i] = m.mean;
+        L->ratio[i] = m.ratio;
+      }
+      t += -(e.k * ::log(m.mean) - m.mean - e.lgk);
     }
     return blk.sum1(t);
   }
+  // the gradient at the point of the last value
   ZEUS_D void gradient(const F& f, const double* th, double* g, bool, Block<NT>& blk)
   {
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
     if constexpr (G == Gradient::Dual) {
+      double t = 0.0; // lane k < 4: derivative k
 #pragma unroll 1
-      for (int i = threadIdx.x; i < f.n; i += NT)
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          v[k] -= f.template bin_log_p<dual::DualNumber>(obj::SeededView{th, k}, i).dual;
-    } else if (f.T != nullptr) {
-      const F::Theta h(th);
-      const double ra = 1.0 / h.a;
-      each_bin(f, [&](const F::Bin& b) { (void)F::bin_gradient(h, ra, b, v); });
+      for (int c0 = 0; c0 < f.n; c0 += NT) {
+        const int i = c0 + int(threadIdx.x);
+        if (i < f.n)
+#pragma unroll 1
+          for (int k = 0; k < 4; ++k)
+            L->dual[k][threadIdx.x] = f.bin_dual(obj::SeededView{th, k}, i).dual;
+        __syncthreads();
+        if (threadIdx.x < 4) {
+          const int n = f.n - c0 < NT ? f.n - c0 : NT;
+#pragma unroll 8
+          for (int j = 0; j < n; ++j)
+            t = t - L->dual[threadIdx.x][j];
+        }
+        __syncthreads();
+      }
+      if (threadIdx.x < 4)
+        g[threadIdx.x] = t;
     } else {
       const double a = th[0], b = th[1], c = th[2], d = th[3];
+      double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
       for (int i = threadIdx.x; i < f.n; i += NT) {
-        const double x = f.P[i];
-        const double k = f.P[f.n + i];
-        const double lx = ::log(x);
-        const double pw = ::pow(1.0 - x, b);
-        const double qw = ::pow(x, c + d * lx);
-        const double mean = a * pw / qw;
-        const double w = 1.0 - k / mean;
-        const double wm = w * mean;
-        v[0] += w * (pw / qw);
-        v[1] += wm * ::log(1.0 - x);
-        v[2] -= wm * lx;
-        v[3] -= wm * (lx * lx);
+        const F::Bin e = bin(f, i);
+        const BinPow m = i < kKeep ? BinPow{L->mean[i], L->ratio[i]}
+                                   : bin_pow(a, b, c, d, e.x, e.t);
+        const double w = 1.0 - e.k / m.mean;
+        const double wm = w * m.mean;
+        v[0] += w * m.ratio;
+        v[1] += wm * (e.t.l1 == e.t.l1 ? e.t.l1 : ::log(1.0 - e.x));
+        v[2] -= wm * e.t.lx;
+        v[3] -= wm * (e.t.lx * e.t.lx);
       }
+      blk.template sum<4>(v);
+      if (threadIdx.x < 4)
+        g[threadIdx.x] = v[threadIdx.x];
     }
-    blk.template sum<4>(v);
-    if (threadIdx.x < 4)
-      g[threadIdx.x] = v[threadIdx.x];
   }
 };
 
@@ -537,78 +556,81 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
       L.x[d] = start_uniform_in(P, uint64_t(sl), d);
   }
   __syncthreads();
-  double bestVal = ev.value(f, L.x, blk);
-  ev.gradient(f, L.x, L.g, true, blk);
-  __syncthreads();
-  for (int i = tid; i < D; i += NT)
-    L.p[i] = -L.g[i];
-  int grads = 1, ls_evals = 0;
+  double bestVal = 0.0, fval = 333777.0, gnorm = 69.0;
+  int grads = 0, ls_evals = 0;
   int status = kStatusUnset;
-  double fval = 333777.0, gnorm = 69.0;
-  int iter = 0;
+  int iter = -1; // the first pass of the loop evaluates the starting point
   bool done = false;
 
+  // One evaluation site for the starting point and every trial: the kernel
+  // holds one copy of the objective's code and of its constants.
   for (; iter < P.max_iter; ++iter) {
-    // trajectory step (bfgs_parallel.cuh:155-166); uniform per workgroup
-    const int64_t to = traj_slot(P.traj, sl, iter);
-    if (to >= 0) {
-      double gg = 0.0;
-      for (int i = tid; i < D; i += NT)
-        gg = ::fma(L.g[i], L.g[i], gg);
-      const double nrm = ::sqrt(blk.sum1(gg));
-      for (int d = tid; d < D; d += NT)
-        P.traj.coords[(int64_t(iter) * D + d) * P.traj.starts + sl] = L.x[d];
-      if (tid == 0) {
-        P.traj.fval[to] = bestVal;
-        P.traj.grad[to] = nrm;
-        P.traj.status[to] = int8_t(kStatusUnset);
+    const bool first = iter < 0;
+    int64_t to = -1;
+    double ddir = 0.0;
+    if (!first) {
+      // trajectory step (bfgs_parallel.cuh:155-166); uniform per workgroup
+      to = traj_slot(P.traj, sl, iter);
+      if (to >= 0) {
+        double gg = 0.0;
+        for (int i = tid; i < D; i += NT)
+          gg = ::fma(L.g[i], L.g[i], gg);
+        const double nrm = ::sqrt(blk.sum1(gg));
+        for (int d = tid; d < D; d += NT)
+          P.traj.coords[(int64_t(iter) * D + d) * P.traj.starts + sl] = L.x[d];
+        if (tid == 0) {
+          P.traj.fval[to] = bestVal;
+          P.traj.grad[to] = nrm;
+          P.traj.status[to] = int8_t(kStatusUnset);
+        }
       }
-    }
-    if (tid == 0)
-      L.flag = load_flag(&ctl->stop_flag);
-    __syncthreads();
-    if (L.flag != 0) {
-      status = kStatusStopped;
-      fval = bestVal;
-      double gg = 0.0;
-      for (int i = tid; i < D; i += NT)
-        gg = ::fma(L.g[i], L.g[i], gg);
-      gnorm = ::sqrt(blk.sum1(gg));
-      done = true;
-      break;
-    }
-    double dd = 0.0;
-    for (int i = tid; i < D; i += NT)
-      dd = ::fma(L.g[i], L.p[i], dd);
-    const double ddir = blk.sum1(dd);
-
-    double alpha = 1.0, f1 = 0.0;
-    bool accepted = false;
-    for (int t = 0; t < kLineSearchTrials; ++t) {
-      for (int j = tid; j < D; j += NT)
-        L.xt[j] = ::fma(alpha, L.p[j], L.x[j]);
+      if (tid == 0)
+        L.flag = load_flag(&ctl->stop_flag);
       __syncthreads();
-      f1 = ev.value(f, L.xt, blk);
-      ++ls_evals;
-      if (f1 <= ::fma(kArmijoC1 * alpha, ddir, bestVal) && f1 < bestVal) {
-        accepted = true;
+      if (L.flag != 0) {
+        status = kStatusStopped;
+        fval = bestVal;
+        double gg = 0.0;
+        for (int i = tid; i < D; i += NT)
+          gg = ::fma(L.g[i], L.g[i], gg);
+        gnorm = ::sqrt(blk.sum1(gg));
+        done = true;
         break;
       }
+      double dd = 0.0;
+      for (int i = tid; i < D; i += NT)
+        dd = ::fma(L.g[i], L.p[i], dd);
+      ddir = blk.sum1(dd);
+    }
+
+    // trials t < 20 at alpha = 2^-t; the point at 2^-20 is taken as it is
+    double alpha = 1.0, fnew = 0.0;
+    for (int t = 0;; ++t) {
+      for (int j = tid; j < D; j += NT)
+        L.xt[j] = first ? L.x[j] : ::fma(alpha, L.p[j], L.x[j]);
+      __syncthreads();
+      fnew = ev.value(f, L.xt, blk);
+      if (first)
+        break;
+      ++ls_evals;
+      if (t == kLineSearchTrials ||
+          (fnew <= ::fma(kArmijoC1 * alpha, ddir, bestVal) && fnew < bestVal))
+        break;
       alpha *= 0.5;
     }
     if (tid == 0 && to >= 0 && P.traj.alpha) // bfgs_parallel.cuh:182-184
       P.traj.alpha[to] = alpha;
-    double fnew = f1;
-    if (!accepted) {
-      for (int j = tid; j < D; j += NT)
-        L.xt[j] = ::fma(alpha, L.p[j], L.x[j]);
-      __syncthreads();
-      fnew = ev.value(f, L.xt, blk);
-      ++ls_evals;
-    }
     ev.gradient(f, L.xt, L.gn, true, blk);
     ++grads;
     __syncthreads();
+    if (first) {
+      bestVal = fnew;
+      for (int i = tid; i < D; i += NT) {
+        L.g[i] = L.gn[i];
+        L.p[i] = -L.gn[i];
+      }
+      continue;
+    }
 
     // v = H' g_new while applying the pending update (one pass over H)
     H.pass(L.gn, sp, ap, pending, L.part);
@@ -718,21 +740,26 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
   __syncthreads();
 }
 
-// Resident workgroups per CU the kernel is compiled for: the MLP with the
-// adjoint gradient alternates evaluation phases (no memory traffic) with the
-// streamed H pass (HBM bound), so two workgroups per CU overlap one's pass
-// with the other's evaluation; the register budget is set for that.
+// Wavefronts per SIMD the kernel is compiled for.  The binned likelihood (one
+// wavefront per start, bound by the issue of its power functions and by their
+// chains): 64 fits of 256 starts took 1.66 ms at four, 1.80 at three and 1.85
+// at two.  The MLP with the adjoint gradient alternates evaluation phases (no
+// memory traffic) with the streamed H pass (HBM bound), so two workgroups per
+// CU overlap one's pass with the other's evaluation; the register budget is
+// set for that.
 template <class F, Gradient G>
-constexpr int group_min_blocks()
+constexpr int group_min_waves()
 {
   if constexpr (requires { F::id; }) // built-in objectives
-    return F::id == obj::kMlp && G == Gradient::Adjoint ? 2 : 1;
+    return F::id == obj::kLogLikelihood                   ? 4
+           : F::id == obj::kMlp && G == Gradient::Adjoint ? 2
+                                                          : 1;
   else
     return 1;
 }
 
 template <class F, int D, int NT, Gradient G, bool HREG, class Prov>
-__global__ __launch_bounds__(NT, (group_min_blocks<F, G>())) void
+__global__ __launch_bounds__(NT, (group_min_waves<F, G>())) void
 bfgs_group_kernel(ClassArgs a, Prov prov)
 {
   __shared__ GroupVectors<D, NT> L;

@@ -7,8 +7,8 @@
 // double-double (the table below), and an evaluation of a bin is one
 // exponential; ln mu, which the Poisson likelihood needs as well, is ln a plus
 // the exponent.  With two powers, two logarithms and a division per bin the
-// evaluation was bound by VALU issue (about 1100 instructions a bin; now about
-// 110).
+// evaluation was bound by VALU issue (two powers of about 270 instructions, two
+// logarithms of about 120; now about 110 in all).
 //
 // Accuracy: the products are kept with their rounding errors (fma) and the
 // exponent is a sum of two doubles, so that mu is off by the rounding of q and
@@ -133,17 +133,31 @@ struct BinMean {
   double ratio; // (1 - x)^b / x^q when !plain
 };
 
-// y^p = exp(h + l) with the limits of the power function; y in (0, 1).
+// y^p = exp(h + l) with the limits of the power function, |h| outside
+// (700, 746); y in (0, 1).
 ZEUS_HD ZEUS_FI double
-pow_limit(double h, double l, double y, double p)
+pow_limit(double h, double l)
 {
-  if (h >= 710.0)
+  if (h > 700.0)
     return __builtin_huge_val();
-  if (h <= -746.0)
+  if (h < -700.0)
     return 0.0;
-  if (::fabs(h) <= 700.0)
-    return exp_sum(h, l);
-  return ::pow(y, p); // about to overflow or denormal, or p is NaN
+  return exp_sum(h, l);
+}
+
+// The power functions themselves, out of line: next to overflow and in the
+// denormal range, for NaN parameters and for bins outside (0, 1).  (Inlined,
+// their constants and temporaries took the fit kernel to one wavefront per
+// SIMD.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__attribute__((noinline))
+#else
+inline
+#endif
+ZEUS_HD DD
+bin_pows(double b, double q, double x)
+{
+  return {::pow(1.0 - x, b), ::pow(x, q)};
 }
 
 // la = log(a); a_plain: a in [1e-30, 1e30].
@@ -155,23 +169,43 @@ bin_mean(double a, double b, double c, double d, double la, bool a_plain, double
   const DD p1 = two_prod(b, t.l1);
   const DD p2 = two_prod(q, t.lx);
   const double r1 = ::fma(b, t.l1_lo, p1.lo), r2 = ::fma(q, t.lx_lo, p2.lo);
+  const DD s = two_sum(p1.hi, -p2.hi);
+  const double lo = s.lo + (r1 - r2);
+  const double h1 = ::fabs(p1.hi), h2 = ::fabs(p2.hi);
   // neither power nor the products with a leave the normal range
-  if (a_plain && ::fabs(p1.hi) <= 300.0 && ::fabs(p2.hi) <= 300.0) {
-    const DD s = two_sum(p1.hi, -p2.hi);
-    const double lo = s.lo + (r1 - r2);
+  if (a_plain && h1 <= 300.0 && h2 <= 300.0) {
     const DD lm = two_sum(la, s.hi);
     return {a * exp_sum(s.hi, lo), lm.hi + (lm.lo + lo), true, 0.0};
   }
-  double pw, qw;
-  if (t.l1 == t.l1) {
-    pw = pow_limit(p1.hi, r1, 1.0 - x, b);
-    qw = pow_limit(p2.hi, r2, x, q);
-  } else {
-    pw = ::pow(1.0 - x, b);
-    qw = ::pow(x, q);
-  }
-  const double mean = a * pw / qw;
-  return {mean, ::log(mean), false, pw / qw};
+  const bool limits = (h1 <= 700.0 || h1 >= 746.0) && (h2 <= 700.0 || h2 >= 746.0);
+  const DD w = limits ? DD{pow_limit(p1.hi, r1), pow_limit(p2.hi, r2)} : bin_pows(b, q, x);
+  const double mean = a * w.hi / w.lo;
+  return {mean, ::log(mean), false, w.hi / w.lo};
+}
+
+// The bin in the fit itself keeps the power functions and their order of
+// operations, so that a fit's trajectory (which the likelihood's flat
+// directions can amplify a rounding error along a million times) does not
+// depend on this file; only powers that are certain to overflow or vanish, as
+// in most trials of a first line search, are not evaluated.
+struct BinPow {
+  double mean, ratio;
+};
+ZEUS_HD ZEUS_FI double
+pow_or_limit(double y, double p, double h) // h = p ln y, rounded; NaN: unknown
+{
+  return h > 711.0 ? __builtin_huge_val() : h < -747.0 ? 0.0 : ::pow(y, p);
+}
+ZEUS_HD ZEUS_FI BinPow
+bin_pow(double a, double b, double c, double d, double x, const BinLogs& t)
+{
+  const double q = c + d * t.lx;
+  const double h1 = b * t.l1;
+  // t.l1 is NaN for a bin outside (0, 1): both powers are evaluated
+  const double h2 = t.l1 == t.l1 ? q * t.lx : t.l1;
+  const double pw = pow_or_limit(1.0 - x, b, h1);
+  const double qw = pow_or_limit(x, q, h2);
+  return {a * pw / qw, pw / qw};
 }
 
 } // namespace zeus::dev

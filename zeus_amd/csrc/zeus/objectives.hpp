@@ -261,7 +261,7 @@ struct Gaussian {
 // parameter block (they do not depend on the parameters being fitted).
 // With the table of the bins' logarithms (binned.hpp, prepared once per call)
 // a double evaluation is one exponential per bin; without it, and in dual
-// numbers, the power functions.
+// numbers, the power functions are evaluated.
 struct LogLikelihood {
   static constexpr std::size_t arity = 4;
   static constexpr int id = kLogLikelihood;
@@ -284,8 +284,11 @@ struct LogLikelihood {
     double x, k, lgk;
     dev::BinLogs t;
   };
+  // without a table, the logarithm NaN of a bin that takes the power functions
   ZEUS_HD Bin bin(int i) const
   {
+    if (T == nullptr)
+      return {P[i], P[n + i], P[2 * n + i], {::log(P[i]), 0.0, __builtin_nan(""), 0.0}};
     return {P[i], P[n + i], P[2 * n + i], {T[i], T[n + i], T[2 * n + i], T[3 * n + i]}};
   }
   ZEUS_HD static double bin_term(const Theta& h, const Bin& v)
@@ -314,35 +317,30 @@ struct LogLikelihood {
     return -(v.k * m.log_mean - m.mean - v.lgk);
   }
 
-  // one bin's contribution in T = double (power functions) or dual numbers
-  template <class T_, class X>
-  ZEUS_HD T_ bin_log_p(const X& th, int i) const
+  // one bin's contribution to the log-likelihood in dual numbers
+  template <class X>
+  ZEUS_HD DualNumber bin_dual(const X& th, int i) const
   {
-    using ::log;
-    using ::pow;
-    using dual::log;
-    using dual::pow;
-    const T_ a = th[0], b = th[1], c = th[2], d = th[3];
-    const T_ x = T_(P[i]);
-    const T_ k = T_(P[n + i]);
-    const T_ mean = a * pow(T_(1.0) - x, b) / pow(x, c + d * log(x));
-    return k * log(mean) - mean - T_(P[2 * n + i]);
+    const DualNumber a = th[0], b = th[1], c = th[2], d = th[3];
+    const DualNumber x = DualNumber(P[i]);
+    const DualNumber k = DualNumber(P[n + i]);
+    const DualNumber mean =
+      a * dual::pow(DualNumber(1.0) - x, b) / dual::pow(x, c + d * dual::log(x));
+    return k * dual::log(mean) - mean - DualNumber(P[2 * n + i]);
   }
   template <class T_, class X>
   ZEUS_HD T_ eval(const X& th) const
   {
     T_ nll = T_(0.0);
     if constexpr (kIsDouble<T_>) {
-      if (T != nullptr) {
-        const double v[4] = {th[0], th[1], th[2], th[3]};
-        const Theta h(v);
-        for (int i = 0; i < n; ++i)
-          nll += bin_term(h, bin(i));
-        return nll;
-      }
+      const double v[4] = {th[0], th[1], th[2], th[3]};
+      const Theta h(v);
+      for (int i = 0; i < n; ++i)
+        nll += bin_term(h, bin(i));
+    } else {
+      for (int i = 0; i < n; ++i)
+        nll -= bin_dual(th, i);
     }
-    for (int i = 0; i < n; ++i)
-      nll -= bin_log_p<T_>(th, i);
     return nll;
   }
   template <class T_>
@@ -353,30 +351,10 @@ struct LogLikelihood {
   ZEUS_HD double value_and_gradient(const double* th, double* g) const
   {
     double nll = 0.0, v[4] = {0.0, 0.0, 0.0, 0.0};
-    if (T != nullptr) {
-      const Theta h(th);
-      const double ra = 1.0 / h.a;
-      for (int i = 0; i < n; ++i)
-        nll += bin_gradient(h, ra, bin(i), v);
-    } else {
-      const double a = th[0], b = th[1], c = th[2], d = th[3];
-      for (int i = 0; i < n; ++i) {
-        const double x = P[i];
-        const double k = P[n + i];
-        const double lx = ::log(x);
-        const double pw = ::pow(1.0 - x, b);
-        const double qw = ::pow(x, c + d * lx);
-        const double mean = a * pw / qw;
-        const double log_p = k * ::log(mean) - mean - P[2 * n + i];
-        nll -= log_p;
-        const double w = 1.0 - k / mean; // d nll / d mean
-        const double wm = w * mean;
-        v[0] += w * (pw / qw);
-        v[1] += wm * ::log(1.0 - x);
-        v[2] -= wm * lx;
-        v[3] -= wm * (lx * lx);
-      }
-    }
+    const Theta h(th);
+    const double ra = 1.0 / h.a;
+    for (int i = 0; i < n; ++i)
+      nll += bin_gradient(h, ra, bin(i), v);
     for (int i = 0; i < 4; ++i)
       g[i] = v[i];
     return nll;

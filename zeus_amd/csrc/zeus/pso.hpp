@@ -421,8 +421,7 @@ struct PsoTeamValue {
       const obj::LogLikelihood::Theta h(x);
       for (int c0 = 0; c0 < f.n; c0 += TS) {
         if (c0 + r < f.n)
-          t[0][r] = f.T != nullptr ? f.bin_term(h, f.bin(c0 + r))
-                                   : -f.template bin_log_p<double>(obj::PtrView{x}, c0 + r);
+          t[0][r] = f.bin_term(h, f.bin(c0 + r));
         team_exchange();
         const int n = f.n - c0 < TS ? f.n - c0 : TS;
 #pragma unroll 8
