@@ -158,18 +158,12 @@ struct GroupEvalSeparable {
         v[1] += ::cos(2.0 * obj::kPi * x[i]);
       }
       blk.template sum<2>(v);
-      const double term1 = -20.0 * ::exp(-0.2 * ::sqrt(v[0] / int(D)));
-      const double term2 = -::exp(v[1] / int(D));
-      return term1 + term2 + 20.0 + ::exp(1.0);
+      return finish(v[0], v[1]);
     } else {
       double t = 0.0;
       for (int i = threadIdx.x; i < D; i += NT)
         t += term(x, i);
-      const double s = blk.sum1(t);
-      if constexpr (F::id == obj::kRastrigin)
-        return 10.0 * D + s;
-      else
-        return s;
+      return finish(blk.sum1(t), 0.0);
     }
   }
   ZEUS_D ZEUS_FI double term(const double* x, int i) const
@@ -185,6 +179,105 @@ struct GroupEvalSeparable {
     } else {
       return x[i] * x[i];
     }
+  }
+  // Line-search trials without a trip through LDS: the values at x + alpha p,
+  // alpha = a0, a0 / 2, ... for kTrials trials side by side.  A lane holds its
+  // coordinates of x and p (and the next coordinate's for Rosenbrock's
+  // coupling) during the search; each trial's terms and sum are value()'s.
+  static constexpr int kTrials = 4;
+  static constexpr int KC = (D + NT - 1) / NT;
+  static constexpr bool kNext = F::id == obj::kRosenbrock;
+  double tx[KC], tp[KC], nx[kNext ? KC : 1], np[kNext ? KC : 1];
+
+  ZEUS_D ZEUS_FI void trials_begin(const double* x, const double* p)
+  {
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+      const int i = int(threadIdx.x) + k * NT;
+      tx[k] = i < D ? x[i] : 0.0;
+      tp[k] = i < D ? p[i] : 0.0;
+      if constexpr (kNext) {
+        nx[k] = i < D - 1 ? x[i + 1] : 0.0;
+        np[k] = i < D - 1 ? p[i + 1] : 0.0;
+      }
+    }
+  }
+  // One trial per lane, for dimensions whose value is a few operations: lane t
+  // takes x + 2^-t p by itself, with the terms added in the pairs of the
+  // wavefront's sum, so the whole search is one evaluation.
+  static constexpr bool kLaneTrials = D <= 4 && NT == kWave;
+  ZEUS_D ZEUS_FI double lane_trial(double alpha, const double* x, const double* p) const
+  {
+    double y[D + 1], u[4] = {0.0, 0.0, 0.0, 0.0}, c[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+      y[i] = ::fma(alpha, p[i], x[i]);
+    y[D] = 0.0;
+#pragma unroll
+    for (int i = 0; i < D && i < 4; ++i) {
+      if constexpr (F::id == obj::kAckley) {
+        u[i] = ::fma(y[i], y[i], u[i]);
+        c[i] += ::cos(2.0 * obj::kPi * y[i]);
+      } else {
+        u[i] += term(y, i);
+      }
+    }
+    const double v = (u[0] + u[1]) + (u[2] + u[3]);
+    return finish(v, (c[0] + c[1]) + (c[2] + c[3]));
+  }
+  // the value from the sum(s) of the terms
+  ZEUS_D ZEUS_FI static double finish(double v, double c)
+  {
+    if constexpr (F::id == obj::kAckley) {
+      const double term1 = -20.0 * ::exp(-0.2 * ::sqrt(v / int(D)));
+      const double term2 = -::exp(c / int(D));
+      return term1 + term2 + 20.0 + ::exp(1.0);
+    } else if constexpr (F::id == obj::kRastrigin) {
+      return 10.0 * D + v;
+    } else {
+      return v;
+    }
+  }
+
+  template <int K>
+  ZEUS_D ZEUS_FI void trials(double a0, double (&v)[K], Block<NT>& blk)
+  {
+    double c[F::id == obj::kAckley ? K : 1] = {};
+#pragma unroll
+    for (int t = 0; t < K; ++t) {
+      const double alpha = a0 * (1.0 / double(1 << t));
+      v[t] = 0.0;
+      if constexpr (F::id == obj::kAckley)
+        c[t] = 0.0;
+#pragma unroll
+      for (int k = 0; k < KC; ++k) {
+        const int i = int(threadIdx.x) + k * NT;
+        const double xi = ::fma(alpha, tp[k], tx[k]);
+        if constexpr (F::id == obj::kRosenbrock) {
+          const double xn = ::fma(alpha, np[k], nx[k]);
+          const double t1 = 1.0 - xi;
+          const double t2 = xn - xi * xi;
+          if (i < D - 1)
+            v[t] += t1 * t1 + 100.0 * t2 * t2;
+        } else if constexpr (F::id == obj::kRastrigin) {
+          if (i < D)
+            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
+        } else if constexpr (F::id == obj::kAckley) {
+          if (i < D) {
+            v[t] = ::fma(xi, xi, v[t]);
+            c[t] += ::cos(2.0 * obj::kPi * xi);
+          }
+        } else if (i < D) {
+          v[t] += xi * xi;
+        }
+      }
+    }
+    blk.template sum<K>(v);
+    if constexpr (F::id == obj::kAckley)
+      blk.template sum<K>(c);
+#pragma unroll
+    for (int t = 0; t < K; ++t)
+      v[t] = finish(v[t], c[F::id == obj::kAckley ? t : 0]);
   }
   ZEUS_D void gradient(const F& f, const double* x, double* g, bool, Block<NT>& blk)
   {
@@ -279,7 +372,7 @@ struct GroupEvalLogLik {
         L->mean[i] = m.mean;
         L->ratio[i] = m.ratio;
       }
-      t += -(e.k * ::log(m.mean) - m.mean - e.lgk);
+      t += F::pow_term(e, m);
     }
     return blk.sum1(t);
   }
@@ -314,12 +407,7 @@ struct GroupEvalLogLik {
         const F::Bin e = bin(f, i);
         const BinPow m = i < kKeep ? BinPow{L->mean[i], L->ratio[i]}
                                    : bin_pow(a, b, c, d, e.x, e.t);
-        const double w = 1.0 - e.k / m.mean;
-        const double wm = w * m.mean;
-        v[0] += w * m.ratio;
-        v[1] += wm * (e.t.l1 == e.t.l1 ? e.t.l1 : ::log(1.0 - e.x));
-        v[2] -= wm * e.t.lx;
-        v[3] -= wm * (e.t.lx * e.t.lx);
+        F::pow_gradient(e, m, v);
       }
       blk.template sum<4>(v);
       if (threadIdx.x < 4)
@@ -519,6 +607,21 @@ struct GroupEvalSelect<obj::Mlp, NT, G> {
   using type = GroupEvalMlp<NT, G>;
 };
 
+// Whether an evaluator takes line-search trials together: 0 one by one through
+// LDS, 1 several side by side (kTrials, a divisor of the 20 after the full
+// step), 2 one per lane.
+template <class Eval>
+constexpr int
+group_batches_trials()
+{
+  if constexpr (requires { Eval::kTrials; }) {
+    static_assert(kLineSearchTrials % Eval::kTrials == 0, "whole batches");
+    return Eval::kLaneTrials ? 2 : 1;
+  } else {
+    return 0;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // LDS vectors of one workgroup.
 template <int D, int NT>
@@ -605,18 +708,62 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
 
     // trials t < 20 at alpha = 2^-t; the point at 2^-20 is taken as it is
     double alpha = 1.0, fnew = 0.0;
+    auto accepts = [&](int t, double a, double v) {
+      return t == kLineSearchTrials ||
+             (v <= ::fma(kArmijoC1 * a, ddir, bestVal) && v < bestVal);
+    };
+    if constexpr (group_batches_trials<Eval>() == 2) {
+      if (!first) { // every trial at once, the first accepted one counts
+        const int t = tid < kLineSearchTrials ? tid : kLineSearchTrials;
+        const double a = ::ldexp(1.0, -t);
+        const double v = ev.lane_trial(a, L.x, L.p);
+        const int pick = __builtin_ctzll(__ballot(accepts(t, a, v)));
+        alpha = ::ldexp(1.0, -pick);
+        fnew = readlane_f64(v, pick);
+        ls_evals += pick + 1;
+      }
+    } else if constexpr (group_batches_trials<Eval>() == 1) {
+      if (!first) {
+        // the full step alone, then four trials at a time (1-4, ... 17-20)
+        ev.trials_begin(L.x, L.p);
+        double v1[1];
+        ev.template trials<1>(1.0, v1, blk);
+        fnew = v1[0];
+        ++ls_evals;
+        bool found = accepts(0, 1.0, fnew);
+#pragma unroll 1
+        for (int t0 = 1; !found; t0 += Eval::kTrials) {
+          double v[Eval::kTrials];
+          const double a0 = alpha * 0.5;
+          ev.template trials<Eval::kTrials>(a0, v, blk);
+#pragma unroll
+          for (int t = 0; t < Eval::kTrials; ++t)
+            if (!found) {
+              alpha = a0 * (1.0 / double(1 << t));
+              fnew = v[t];
+              ++ls_evals;
+              found = accepts(t0 + t, alpha, fnew);
+            }
+        }
+      }
+    }
     for (int t = 0;; ++t) {
       for (int j = tid; j < D; j += NT)
         L.xt[j] = first ? L.x[j] : ::fma(alpha, L.p[j], L.x[j]);
       __syncthreads();
-      fnew = ev.value(f, L.xt, blk);
-      if (first)
+      if constexpr (group_batches_trials<Eval>() != 0) {
+        if (first)
+          fnew = ev.value(f, L.xt, blk);
         break;
-      ++ls_evals;
-      if (t == kLineSearchTrials ||
-          (fnew <= ::fma(kArmijoC1 * alpha, ddir, bestVal) && fnew < bestVal))
-        break;
-      alpha *= 0.5;
+      } else {
+        fnew = ev.value(f, L.xt, blk);
+        if (first)
+          break;
+        ++ls_evals;
+        if (accepts(t, alpha, fnew))
+          break;
+        alpha *= 0.5;
+      }
     }
     if (tid == 0 && to >= 0 && P.traj.alpha) // bfgs_parallel.cuh:182-184
       P.traj.alpha[to] = alpha;

@@ -260,8 +260,8 @@ struct Gaussian {
 // - lgamma(k_i + 1)].  The lgamma(k+1) constants come precomputed in the
 // parameter block (they do not depend on the parameters being fitted).
 // With the table of the bins' logarithms (binned.hpp, prepared once per call)
-// a double evaluation is one exponential per bin; without it, and in dual
-// numbers, the power functions are evaluated.
+// a bin can be evaluated by one exponential (bin_term, bin_gradient: the swarm
+// and zeus_eval); the fits keep the power functions (bin_pow).
 struct LogLikelihood {
   static constexpr std::size_t arity = 4;
   static constexpr int id = kLogLikelihood;
@@ -328,15 +328,30 @@ struct LogLikelihood {
       a * dual::pow(DualNumber(1.0) - x, b) / dual::pow(x, c + d * dual::log(x));
     return k * dual::log(mean) - mean - DualNumber(P[2 * n + i]);
   }
+  // one bin's value and gradient terms from its mean by power functions
+  ZEUS_HD static double pow_term(const Bin& e, const dev::BinPow& m)
+  {
+    return -(e.k * ::log(m.mean) - m.mean - e.lgk);
+  }
+  ZEUS_HD static void pow_gradient(const Bin& e, const dev::BinPow& m, double (&g)[4])
+  {
+    const double w = 1.0 - e.k / m.mean; // d nll / d mean
+    const double wm = w * m.mean;
+    g[0] += w * m.ratio;
+    // ln(1 - x) is NaN where both powers are evaluated
+    g[1] += wm * (e.t.l1 == e.t.l1 ? e.t.l1 : ::log(1.0 - e.x));
+    g[2] -= wm * e.t.lx;
+    g[3] -= wm * (e.t.lx * e.t.lx);
+  }
   template <class T_, class X>
   ZEUS_HD T_ eval(const X& th) const
   {
     T_ nll = T_(0.0);
     if constexpr (kIsDouble<T_>) {
-      const double v[4] = {th[0], th[1], th[2], th[3]};
-      const Theta h(v);
-      for (int i = 0; i < n; ++i)
-        nll += bin_term(h, bin(i));
+      for (int i = 0; i < n; ++i) {
+        const Bin e = bin(i);
+        nll += pow_term(e, dev::bin_pow(th[0], th[1], th[2], th[3], e.x, e.t));
+      }
     } else {
       for (int i = 0; i < n; ++i)
         nll -= bin_dual(th, i);
@@ -351,10 +366,12 @@ struct LogLikelihood {
   ZEUS_HD double value_and_gradient(const double* th, double* g) const
   {
     double nll = 0.0, v[4] = {0.0, 0.0, 0.0, 0.0};
-    const Theta h(th);
-    const double ra = 1.0 / h.a;
-    for (int i = 0; i < n; ++i)
-      nll += bin_gradient(h, ra, bin(i), v);
+    for (int i = 0; i < n; ++i) {
+      const Bin e = bin(i);
+      const dev::BinPow m = dev::bin_pow(th[0], th[1], th[2], th[3], e.x, e.t);
+      nll += pow_term(e, m);
+      pow_gradient(e, m, v);
+    }
     for (int i = 0; i < 4; ++i)
       g[i] = v[i];
     return nll;
