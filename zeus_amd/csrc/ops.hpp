@@ -4,6 +4,8 @@
 
 #include "runtime.hpp"
 
+#include <algorithm>
+
 namespace zeus::rt {
 
 template <class F, int D, Gradient G>
@@ -17,6 +19,47 @@ eval_kernel(dev::ProblemDesc P, const double* x, int64_t n, double* f, double* g
   f[i] = dev::lane_value<F, D>(fn, x + i * D);
   if (g)
     dev::lane_gradient<F, D, G>(fn, x + i * D, g + i * D);
+}
+
+// Values and gradients of the binned likelihood: a team of 16 lanes per point
+// splits the bins.  A lane per point walked 100 bins with the power functions
+// on 250 wavefronts for 16000 points (254 us, value and gradient in two
+// passes); the teams make one pass over 4000 wavefronts.
+constexpr int kEvalTeam = 16, kEvalTeams = 256 / kEvalTeam;
+
+template <Gradient G>
+__global__ __launch_bounds__(256) void
+eval_bins_kernel(dev::ProblemDesc P, const double* x, int64_t n, double* f, double* g)
+{
+  using F = obj::LogLikelihood;
+  const int r = threadIdx.x % kEvalTeam;
+  const F fn = dev::BuiltinProvider{}.template get<F>(P);
+  const bool adjoint = g != nullptr && G == Gradient::Adjoint;
+  for (int64_t i = int64_t(blockIdx.x) * kEvalTeams + threadIdx.x / kEvalTeam; i < n;
+       i += int64_t(gridDim.x) * kEvalTeams) {
+    const double th[4] = {x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+    const F::Theta h(th);
+    const double ra = 1.0 / h.a;
+    double v = 0.0, d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int b = r; b < fn.n; b += kEvalTeam) {
+      const F::Bin e = fn.bin(b);
+      v += adjoint ? F::bin_gradient(h, ra, e, d) : F::bin_term(h, e);
+      if constexpr (G == Gradient::Dual)
+        if (g != nullptr)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            d[k] -= fn.bin_dual(obj::SeededView{th, k}, b).dual;
+    }
+    v = dev::team_sum<kEvalTeam>(v);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      d[k] = dev::team_sum<kEvalTeam>(d[k]);
+    if (r == 0)
+      f[i] = v;
+    if (g != nullptr && r < 4)
+      g[4 * i + r] = r == 0 ? d[0] : r == 1 ? d[1] : r == 2 ? d[2] : d[3];
+  }
 }
 
 template <class F, int D>
@@ -274,11 +317,20 @@ struct Ops {
     const int nb = int((n + 127) / 128);
     if (nb == 0)
       return hipSuccess;
-    if (gradient == 1)
-      eval_kernel<F, D, Gradient::Dual><<<nb, 128, 0, s>>>(P, x, n, f, g);
-    else
-      eval_kernel<F, D, Gradient::Adjoint><<<nb, 128, 0, s>>>(P, x, n, f, g);
-    return hipGetLastError();
+    if constexpr (F::id == obj::kLogLikelihood) {
+      const int grid = int(std::min<int64_t>((n + kEvalTeams - 1) / kEvalTeams, 1 << 20));
+      if (gradient == 1)
+        eval_bins_kernel<Gradient::Dual><<<grid, 256, 0, s>>>(P, x, n, f, g);
+      else
+        eval_bins_kernel<Gradient::Adjoint><<<grid, 256, 0, s>>>(P, x, n, f, g);
+      return hipGetLastError();
+    } else {
+      if (gradient == 1)
+        eval_kernel<F, D, Gradient::Dual><<<nb, 128, 0, s>>>(P, x, n, f, g);
+      else
+        eval_kernel<F, D, Gradient::Adjoint><<<nb, 128, 0, s>>>(P, x, n, f, g);
+      return hipGetLastError();
+    }
   }
 
   static const ClassOps* table()
