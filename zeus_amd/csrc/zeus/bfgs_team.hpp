@@ -126,6 +126,57 @@ struct TeamEval {
     }
   }
 
+  // Values at x + alpha p, alpha = a0, a0 / 2, ... for K trials side by side,
+  // from the lane's own coordinates x and p (and the next coordinate's, nx and
+  // np, for Rosenbrock's coupling): value()'s terms and sums, no LDS.
+  static constexpr bool kNext = F::id == obj::kRosenbrock;
+  template <int K>
+  ZEUS_D ZEUS_FI static void trials(double a0, int r, const double (&x)[KC],
+                                    const double (&p)[KC], const double (&nx)[KC],
+                                    const double (&np)[KC], double (&v)[K])
+  {
+    double c[K];
+#pragma unroll
+    for (int t = 0; t < K; ++t) {
+      const double alpha = a0 * (1.0 / double(1 << t));
+      v[t] = c[t] = 0.0;
+#pragma unroll
+      for (int k = 0; k < KC; ++k) {
+        const int i = r + TS * k;
+        const double xi = ::fma(alpha, p[k], x[k]);
+        if constexpr (F::id == obj::kRosenbrock) {
+          const double xn = ::fma(alpha, np[k], nx[k]);
+          const double t1 = 1.0 - xi;
+          const double t2 = xn - xi * xi;
+          if (i < D - 1)
+            v[t] += t1 * t1 + 100.0 * t2 * t2;
+        } else if constexpr (F::id == obj::kRastrigin) {
+          if (i < D)
+            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
+        } else if constexpr (F::id == obj::kAckley) {
+          if (i < D) {
+            v[t] = ::fma(xi, xi, v[t]);
+            c[t] += ::cos(2.0 * obj::kPi * xi);
+          }
+        } else if (i < D) {
+          v[t] += xi * xi;
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < K; ++t) {
+      v[t] = team_sum<TS>(v[t]);
+      if constexpr (F::id == obj::kAckley) {
+        c[t] = team_sum<TS>(c[t]);
+        const double term1 = -20.0 * ::exp(-0.2 * ::sqrt(v[t] / int(D)));
+        const double term2 = -::exp(c[t] / int(D));
+        v[t] = term1 + term2 + 20.0 + ::exp(1.0);
+      } else if constexpr (F::id == obj::kRastrigin) {
+        v[t] = 10.0 * D + v[t];
+      }
+    }
+  }
+
   template <Gradient G>
   ZEUS_D static void gradient(const F& f, const double* xl, int r, double (&g)[KC])
   {
@@ -201,6 +252,10 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
   constexpr int KC = (D + TS - 1) / TS;
   constexpr int kTeams = kTeamThreads / TS;
   using E = TeamEval<F, D, TS>;
+  // line-search trials side by side (the Ackley value ends in two exponentials
+  // and a square root, which do not interleave)
+  constexpr int kTrials = F::id == obj::kAckley ? 1 : 4;
+  static_assert(kLineSearchTrials % kTrials == 0, "whole batches");
   // per team: the point being evaluated, and the new gradient and pending
   // pair broadcast for the H pass
   __shared__ double lds_x[kTeams][D];
@@ -294,25 +349,50 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
         break;
       }
       const double ddir = dot(g, p);
-      double alpha = 1.0, f1 = 0.0;
-      bool accepted = false;
-      for (int t = 0; t < kLineSearchTrials; ++t) {
-        stage_trial(alpha);
-        f1 = E::value(xl, r);
-        ++ls_evals;
-        if (f1 <= ::fma(kArmijoC1 * alpha, ddir, bestVal) && f1 < bestVal) {
-          accepted = true;
-          break;
+      // the neighbours' coordinates for the search, through the slots that
+      // carry the rank-2 pair later
+      double nx[KC], np[KC];
+      if constexpr (E::kNext) {
+        stage(x, sb);
+        stage(p, ab);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+          const int i = r + TS * k;
+          nx[k] = i < D - 1 ? sb[i + 1] : 0.0;
+          np[k] = i < D - 1 ? ab[i + 1] : 0.0;
         }
-        alpha *= 0.5;
-        team_exchange();
+      } else {
+#pragma unroll
+        for (int k = 0; k < KC; ++k)
+          nx[k] = np[k] = 0.0;
       }
-      double fnew = f1;
-      if (!accepted) {
-        stage_trial(alpha);
-        fnew = E::value(xl, r);
+      // trials t < 20 at alpha = 2^-t, the full step alone, then kTrials at a
+      // time; the point at 2^-20 is taken as it is
+      double alpha = 1.0, fnew;
+      bool found;
+      {
+        double v[1];
+        E::template trials<1>(1.0, r, x, p, nx, np, v);
+        fnew = v[0];
         ++ls_evals;
+        found = fnew <= ::fma(kArmijoC1, ddir, bestVal) && fnew < bestVal;
       }
+#pragma unroll 1
+      for (int t0 = 1; !found; t0 += kTrials) {
+        double v[kTrials];
+        const double a0 = alpha * 0.5;
+        E::template trials<kTrials>(a0, r, x, p, nx, np, v);
+#pragma unroll
+        for (int t = 0; t < kTrials; ++t)
+          if (!found) {
+            alpha = a0 * (1.0 / double(1 << t));
+            fnew = v[t];
+            ++ls_evals;
+            found = t0 + t == kLineSearchTrials ||
+                    (fnew <= ::fma(kArmijoC1 * alpha, ddir, bestVal) && fnew < bestVal);
+          }
+      }
+      stage_trial(alpha);
       E::template gradient<G>(f, xl, r, gn);
       ++grads;
 
