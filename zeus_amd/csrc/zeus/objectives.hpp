@@ -21,6 +21,7 @@
 #include "binned.hpp"
 #include "dual.hpp"
 #include "traits.hpp"
+#include "trig.hpp"
 
 #include <array>
 #include <cmath>
@@ -123,15 +124,34 @@ struct Rastrigin {
   const double* zeus_params() const { return nullptr; }
   long long zeus_n_params() const { return 0; }
 
+  // cos(2 pi x) and sin(2 pi x): beyond four dimensions by turns (trig.hpp),
+  // where the value and every trial of a line search are D of them; up to four
+  // the library's functions, whose cost the launches hide
+  ZEUS_HD static double cosine(double x)
+  {
+    if constexpr (D > 4)
+      return dev::cos_turns(x);
+    else
+      return ::cos(2.0 * kPi * x);
+  }
+  ZEUS_HD static double sine(double x)
+  {
+    if constexpr (D > 4)
+      return dev::sin_turns(x);
+    else
+      return ::sin(2.0 * kPi * x);
+  }
+
   template <class T, class X>
   ZEUS_HD T eval(const X& x) const
   {
-    using ::cos;
-    using dual::cos;
     T sum = T(10.0 * D);
     for (int i = 0; i < int(D); ++i) {
       const T xi = x[i];
-      sum = sum + (xi * xi - T(10.0) * cos(xi * T(2.0 * kPi)));
+      if constexpr (kIsDouble<T>)
+        sum = sum + (xi * xi - 10.0 * cosine(xi));
+      else
+        sum = sum + (xi * xi - T(10.0) * dual::cos(xi * T(2.0 * kPi)));
     }
     return sum;
   }
@@ -145,9 +165,8 @@ struct Rastrigin {
     const double k = 10.0 * (2.0 * kPi);
     double sum = 10.0 * D;
     for (int i = 0; i < int(D); ++i) {
-      const double w = 2.0 * kPi * x[i];
-      sum += x[i] * x[i] - 10.0 * ::cos(w);
-      g[i] = 2.0 * x[i] + k * ::sin(w);
+      sum += x[i] * x[i] - 10.0 * cosine(x[i]);
+      g[i] = 2.0 * x[i] + k * sine(x[i]);
     }
     return sum;
   }
