@@ -150,6 +150,13 @@ load_flag(const int32_t* p)
 {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Whether a problem can stop early at all: an iteration that cannot be stopped
+// does not wait for the flag (a device-scope load, close to a microsecond).
+ZEUS_D ZEUS_FI bool
+may_stop(const ProblemDesc& P)
+{
+  return P.required > 0 && P.required <= P.n_starts;
+}
 ZEUS_D ZEUS_FI void
 store_flag(int32_t* p, int v)
 {

@@ -331,6 +331,7 @@ struct GroupEvalSeparable {
 template <int NT, Gradient G>
 struct GroupEvalLogLik {
   using F = obj::LogLikelihood;
+  static constexpr bool kOneSite = true;
   static constexpr int kKeep = 128;
   static constexpr int kFields = 5; // x, k, lgamma(k + 1), ln x, ln(1 - x)
   struct Lds {
@@ -622,6 +623,15 @@ group_batches_trials()
   }
 }
 
+// Whether the kernel evaluates starting points and trials at one place in its
+// code (the binned likelihood's four power functions per pair of bins).
+template <class Eval>
+constexpr bool
+group_one_site()
+{
+  return requires { Eval::kOneSite; };
+}
+
 // ---------------------------------------------------------------------------
 // LDS vectors of one workgroup.
 template <int D, int NT>
@@ -662,13 +672,24 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
   double bestVal = 0.0, fval = 333777.0, gnorm = 69.0;
   int grads = 0, ls_evals = 0;
   int status = kStatusUnset;
-  int iter = -1; // the first pass of the loop evaluates the starting point
   bool done = false;
+  const bool stoppable = may_stop(P);
+  // One evaluation site for the starting point and every trial (kOneSite: the
+  // first pass of the loop evaluates the starting point) keeps one copy of a
+  // large objective's code and constants in the kernel.
+  constexpr bool kOneSite = group_one_site<Eval>();
+  int iter = kOneSite ? -1 : 0;
+  if constexpr (!kOneSite) {
+    bestVal = ev.value(f, L.x, blk);
+    ev.gradient(f, L.x, L.g, true, blk);
+    ++grads;
+    __syncthreads();
+    for (int i = tid; i < D; i += NT)
+      L.p[i] = -L.g[i];
+  }
 
-  // One evaluation site for the starting point and every trial: the kernel
-  // holds one copy of the objective's code and of its constants.
   for (; iter < P.max_iter; ++iter) {
-    const bool first = iter < 0;
+    const bool first = kOneSite && iter < 0;
     int64_t to = -1;
     double ddir = 0.0;
     if (!first) {
@@ -687,10 +708,14 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
           P.traj.status[to] = int8_t(kStatusUnset);
         }
       }
-      if (tid == 0)
-        L.flag = load_flag(&ctl->stop_flag);
-      __syncthreads();
-      if (L.flag != 0) {
+      bool stop = false; // uniform per workgroup
+      if (stoppable) {
+        if (tid == 0)
+          L.flag = load_flag(&ctl->stop_flag);
+        __syncthreads();
+        stop = L.flag != 0;
+      }
+      if (stop) {
         status = kStatusStopped;
         fval = bestVal;
         double gg = 0.0;
@@ -713,49 +738,46 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
              (v <= ::fma(kArmijoC1 * a, ddir, bestVal) && v < bestVal);
     };
     if constexpr (group_batches_trials<Eval>() == 2) {
-      if (!first) { // every trial at once, the first accepted one counts
-        const int t = tid < kLineSearchTrials ? tid : kLineSearchTrials;
-        const double a = ::ldexp(1.0, -t);
-        const double v = ev.lane_trial(a, L.x, L.p);
-        const int pick = __builtin_ctzll(__ballot(accepts(t, a, v)));
-        alpha = ::ldexp(1.0, -pick);
-        fnew = readlane_f64(v, pick);
-        ls_evals += pick + 1;
-      }
+      // every trial at once, the first accepted one counts
+      const int t = tid < kLineSearchTrials ? tid : kLineSearchTrials;
+      const double a = ::ldexp(1.0, -t);
+      const double v = ev.lane_trial(a, L.x, L.p);
+      const int pick = __builtin_ctzll(__ballot(accepts(t, a, v)));
+      alpha = ::ldexp(1.0, -pick);
+      fnew = readlane_f64(v, pick);
+      ls_evals += pick + 1;
     } else if constexpr (group_batches_trials<Eval>() == 1) {
-      if (!first) {
-        // the full step alone, then four trials at a time (1-4, ... 17-20)
-        ev.trials_begin(L.x, L.p);
-        double v1[1];
-        ev.template trials<1>(1.0, v1, blk);
-        fnew = v1[0];
-        ++ls_evals;
-        bool found = accepts(0, 1.0, fnew);
+      // the full step alone, then four trials at a time (1-4, ... 17-20)
+      ev.trials_begin(L.x, L.p);
+      double v1[1];
+      ev.template trials<1>(1.0, v1, blk);
+      fnew = v1[0];
+      ++ls_evals;
+      bool found = accepts(0, 1.0, fnew);
 #pragma unroll 1
-        for (int t0 = 1; !found; t0 += Eval::kTrials) {
-          double v[Eval::kTrials];
-          const double a0 = alpha * 0.5;
-          ev.template trials<Eval::kTrials>(a0, v, blk);
+      for (int t0 = 1; !found; t0 += Eval::kTrials) {
+        double v[Eval::kTrials];
+        const double a0 = alpha * 0.5;
+        ev.template trials<Eval::kTrials>(a0, v, blk);
 #pragma unroll
-          for (int t = 0; t < Eval::kTrials; ++t)
-            if (!found) {
-              alpha = a0 * (1.0 / double(1 << t));
-              fnew = v[t];
-              ++ls_evals;
-              found = accepts(t0 + t, alpha, fnew);
-            }
-        }
+        for (int t = 0; t < Eval::kTrials; ++t)
+          if (!found) {
+            alpha = a0 * (1.0 / double(1 << t));
+            fnew = v[t];
+            ++ls_evals;
+            found = accepts(t0 + t, alpha, fnew);
+          }
       }
     }
-    for (int t = 0;; ++t) {
+    if constexpr (group_batches_trials<Eval>() != 0) {
       for (int j = tid; j < D; j += NT)
-        L.xt[j] = first ? L.x[j] : ::fma(alpha, L.p[j], L.x[j]);
+        L.xt[j] = ::fma(alpha, L.p[j], L.x[j]);
       __syncthreads();
-      if constexpr (group_batches_trials<Eval>() != 0) {
-        if (first)
-          fnew = ev.value(f, L.xt, blk);
-        break;
-      } else {
+    } else if constexpr (kOneSite) {
+      for (int t = 0;; ++t) {
+        for (int j = tid; j < D; j += NT)
+          L.xt[j] = first ? L.x[j] : ::fma(alpha, L.p[j], L.x[j]);
+        __syncthreads();
         fnew = ev.value(f, L.xt, blk);
         if (first)
           break;
@@ -763,6 +785,27 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
         if (accepts(t, alpha, fnew))
           break;
         alpha *= 0.5;
+      }
+    } else {
+      bool accepted = false;
+      for (int t = 0; t < kLineSearchTrials; ++t) {
+        for (int j = tid; j < D; j += NT)
+          L.xt[j] = ::fma(alpha, L.p[j], L.x[j]);
+        __syncthreads();
+        fnew = ev.value(f, L.xt, blk);
+        ++ls_evals;
+        if (accepts(t, alpha, fnew)) {
+          accepted = true;
+          break;
+        }
+        alpha *= 0.5;
+      }
+      if (!accepted) {
+        for (int j = tid; j < D; j += NT)
+          L.xt[j] = ::fma(alpha, L.p[j], L.x[j]);
+        __syncthreads();
+        fnew = ev.value(f, L.xt, blk);
+        ++ls_evals;
       }
     }
     if (tid == 0 && to >= 0 && P.traj.alpha) // bfgs_parallel.cuh:182-184

@@ -275,6 +275,7 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
     Control* ctl = a.ctl + pi;
     decltype(auto) f = prov.template get<F>(P);
     const int64_t sl = s - P.start0;
+    const bool stoppable = may_stop(P);
 
     double x[KC], g[KC], p[KC], gn[KC]; // the trial point lives in LDS (xl)
     double H[KC][D];
@@ -341,7 +342,7 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
 
     for (; iter < P.max_iter; ++iter) {
       team_exchange(); // the previous evaluation's reads of xl are done
-      if (load_flag(&ctl->stop_flag) != 0) {
+      if (stoppable && load_flag(&ctl->stop_flag) != 0) {
         status = kStatusStopped;
         fval = bestVal;
         gnorm = ::sqrt(dot(g, g));

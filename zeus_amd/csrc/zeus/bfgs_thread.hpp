@@ -59,6 +59,7 @@ thread_bfgs(const F& f, const ProblemDesc& P, Control* ctl, int64_t s,
 {
   constexpr int kU = D <= kThreadRegMaxD ? D : 1; // unroll factor
   const int64_t sl = s - P.start0; // start index within its problem
+  const bool stoppable = may_stop(P);
   // timing (bfgs_sequential.cuh:50,86-97,149-173,222-232), when requested
   const bool timed = out.ad_ticks != nullptr;
   const uint64_t k_begin = timed ? uint64_t(wall_clock64()) : 0;
@@ -116,7 +117,7 @@ thread_bfgs(const F& f, const ProblemDesc& P, Control* ctl, int64_t s,
       P.traj.status[to] = int8_t(kStatusUnset);
     }
     // stop flag raised by another start (bfgs_common.cuh:115-141)
-    if (load_flag(&ctl->stop_flag) != 0) {
+    if (stoppable && load_flag(&ctl->stop_flag) != 0) {
       status = kStatusStopped;
       fval = bestVal; // == f(x): x is where bestVal was evaluated
       double gg = 0.0;

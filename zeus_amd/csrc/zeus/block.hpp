@@ -146,6 +146,19 @@ struct Block {
 #pragma unroll
     for (int k = 0; k < K; ++k)
       v[k] = wave_sum(v[k]);
+    if constexpr (kWaves == 1) {
+      // every lane has the wavefront's sum already: no trip through LDS (0.0 +
+      // as the fold below starts).  The wavefront's LDS operations complete in
+      // order; the fences keep the compiler from moving a caller's LDS accesses
+      // across, as the barrier does for more wavefronts.
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        v[k] = 0.0 + v[k];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      return;
+    }
     double* r = red + parity * (4 * kWaves);
     parity ^= 1;
     const int w = threadIdx.x / kWave;
