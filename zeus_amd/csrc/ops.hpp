@@ -266,7 +266,7 @@ struct Ops {
   template <int NT>
   static constexpr int64_t slab_doubles()
   {
-    return kHReg<NT> ? 0 : int64_t(dev::RowChunk<D, NT>::kPerThread) * NT;
+    return dev::group_slab_doubles<D, NT, kHReg<NT>>();
   }
   static int64_t group_slab_per_block(int nt)
   {

@@ -634,11 +634,12 @@ group_one_site()
 
 // ---------------------------------------------------------------------------
 // LDS vectors of one workgroup.
-template <int D, int NT>
+template <int D, int NT, bool PAIRS>
 struct GroupVectors {
   double x[D], g[D], p[D], xt[D], gn[D], v[D];
-  double s0[D], a0[D], s1[D], a1[D]; // current / pending rank-2 pair
-  double part[RowChunk<D, NT>::CH * D];
+  double s0[D], a0[D]; // current rank-2 pair
+  double s1[PAIRS ? 1 : D], a1[PAIRS ? 1 : D]; // pending one (none with a pair list)
+  double part[PAIRS ? pair_parts<D, NT>() * D : RowChunk<D, NT>::CH * D];
   double stash[D];
   double red[8 * (NT / kWave)];
   double scalar[4];
@@ -647,12 +648,14 @@ struct GroupVectors {
 
 template <class F, int D, int NT, Gradient G, bool HREG, class Eval>
 ZEUS_D void
-group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval& ev,
+group_bfgs(const F& f, GroupVectors<D, NT, kPairForm<D, NT, HREG>>& L,
+           GroupH<D, NT, HREG>& H, Eval& ev,
            Block<NT>& blk, const ProblemDesc& P, Control* ctl, int64_t s,
            const double* starts, const StartOut& out)
 {
   const int tid = threadIdx.x;
   const int64_t sl = s - P.start0;
+  constexpr bool kPairs = kPairForm<D, NT, HREG>;
   double* sc = L.s0; // s of this iteration
   double* ac = L.a0;
   double* sp = L.s1; // pending pair from the previous iteration
@@ -822,12 +825,21 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
       continue;
     }
 
-    // v = H' g_new while applying the pending update (one pass over H)
-    H.pass(L.gn, sp, ap, pending, L.part);
-    __syncthreads();
+    // v = H' g_new: from the pairs, or while applying the pending update (one
+    // pass over H)
+    if constexpr (kPairs) {
+      H.apply(L.gn, L.part);
+    } else {
+      H.pass(L.gn, sp, ap, pending, L.part);
+      __syncthreads();
+    }
     double st[2] = {0.0, 0.0};
     for (int i = tid; i < D; i += NT) {
-      const double v = chunk_total<D, NT>(L.part, i);
+      double v;
+      if constexpr (kPairs)
+        v = H.total(L.part, L.gn, i);
+      else
+        v = chunk_total<D, NT>(L.part, i);
       L.v[i] = v;
       const double si = L.xt[i] - L.x[i];
       const double yi = L.gn[i] - L.g[i];
@@ -857,6 +869,8 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
         const double hg = acc ? L.v[i] : -L.p[i];
         L.p[i] = -::fma(ac[i], q[1], ::fma(sc[i], q[0], hg));
       }
+      if constexpr (kPairs)
+        H.append(sc, ac);
     } else {
       for (int i = tid; i < D; i += NT)
         L.p[i] = acc ? -L.v[i] : L.p[i];
@@ -872,14 +886,15 @@ group_bfgs(const F& f, GroupVectors<D, NT>& L, DistMatrix<D, NT, HREG>& H, Eval&
     for (int i = tid; i < D; i += NT)
       gg = ::fma(L.g[i], L.g[i], gg);
     const double nrm = ::sqrt(blk.sum1(gg));
-    // the new pair becomes pending for the next pass
-    pending = upd;
-    double* t0 = sp;
-    double* t1 = ap;
-    sp = sc;
-    ap = ac;
-    sc = t0;
-    ac = t1;
+    if constexpr (!kPairs) { // the new pair becomes pending for the next pass
+      pending = upd;
+      double* t0 = sp;
+      double* t1 = ap;
+      sp = sc;
+      ap = ac;
+      sc = t0;
+      ac = t1;
+    }
 
     if (!::isfinite(nrm) || !::isfinite(fnew)) {
       status = kStatusNonFinite;
@@ -952,13 +967,13 @@ template <class F, int D, int NT, Gradient G, bool HREG, class Prov>
 __global__ __launch_bounds__(NT, (group_min_waves<F, G>())) void
 bfgs_group_kernel(ClassArgs a, Prov prov)
 {
-  __shared__ GroupVectors<D, NT> L;
+  __shared__ GroupVectors<D, NT, kPairForm<D, NT, HREG>> L;
   Block<NT> blk{L.red};
   using Eval = typename GroupEvalSelect<F, NT, G>::type;
   static_assert(int(F::arity) == D, "objective arity and kernel dimension differ");
   Eval ev;
   ev.sc = GroupScratch{L.part, L.stash, L.scalar};
-  DistMatrix<D, NT, HREG> H;
+  GroupH<D, NT, HREG> H;
   if constexpr (!HREG)
     H.slab = a.h_slab + int64_t(blockIdx.x) * a.h_slab_stride;
   int bound = -1;

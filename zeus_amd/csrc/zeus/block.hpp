@@ -3,6 +3,8 @@
 
 #include "config.hpp"
 
+#include <type_traits>
+
 namespace zeus::dev {
 
 // One DPP lane exchange of a double (two 32-bit moves).  Every pattern used
@@ -203,6 +205,7 @@ struct RowChunk {
 // element e of thread t sits at slab[e * NT + t] (coalesced).
 template <int D, int NT, bool REG>
 struct DistMatrix {
+  static constexpr bool kPairs = false;
   using Lay = RowChunk<D, NT>;
   double m[REG ? Lay::kPerThread : 1];
   double* slab = nullptr;
@@ -251,20 +254,6 @@ struct DistMatrix {
   ZEUS_D ZEUS_FI void pass(const double* x, const double* s, const double* a,
                            bool pending, double* part)
   {
-    if constexpr (!REG && D > 256) {
-      if (pending)
-        pass_slab<true>(x, s, a, part);
-      else
-        pass_slab<false>(x, s, a, part);
-    } else {
-      pass_regs(x, s, a, pending, part);
-    }
-  }
-
-  // Register form, and slab form for rows up to 256 elements.
-  ZEUS_D ZEUS_FI void pass_regs(const double* x, const double* s, const double* a,
-                                bool pending, double* part)
-  {
     const int c = threadIdx.x % Lay::CH, r0 = threadIdx.x / Lay::CH;
 #pragma unroll(REG ? 64 : 1)
     for (int k = 0; k < Lay::R; ++k) {
@@ -289,71 +278,6 @@ struct DistMatrix {
       }
     }
   }
-
-  // Slab form of pass() for long rows (D > 256): the same arithmetic in the
-  // same order, with the columns taken in batches of kBatch whose slab loads
-  // are all issued before any of them is used (a branch per element would
-  // wait out the memory latency element by element, and at these sizes one
-  // wave per SIMD has no other wave to hide it; measured 2x on the 321-D
-  // MLP).  Shorter rows keep the element loop of pass_regs, which leaves
-  // registers for more resident waves (measured faster at D = 150).  Padding
-  // columns (col >= D) are loaded but neither updated nor summed.
-  template <bool PENDING>
-  ZEUS_D ZEUS_FI void pass_slab(const double* x, const double* s, const double* a, double* part)
-  {
-    constexpr int kBatch = 16;
-    const int c = threadIdx.x % Lay::CH, r0 = threadIdx.x / Lay::CH;
-    double* base = slab + threadIdx.x;
-    for (int k = 0; k < Lay::R; ++k) {
-      const int row = r0 + k * Lay::RPP;
-      if (row >= D)
-        continue;
-      const double sr = PENDING ? s[row] : 0.0;
-      const double ar = PENDING ? a[row] : 0.0;
-      double* hrow = base + int64_t(k) * Lay::L * NT;
-      double acc = 0.0;
-      int l0 = 0;
-      // one batch per step: unrolled further, the loads of every batch are
-      // hoisted together and the register count (and occupancy) suffers
-#pragma unroll 1
-      for (; l0 + kBatch <= Lay::L; l0 += kBatch) {
-        double h[kBatch];
-#pragma unroll
-        for (int i = 0; i < kBatch; ++i)
-          h[i] = hrow[int64_t(l0 + i) * NT];
-#pragma unroll
-        for (int i = 0; i < kBatch; ++i) {
-          const int col = c * Lay::L + l0 + i;
-          const bool ok = col < D;
-          const int cc = ok ? col : D - 1;
-          if constexpr (PENDING) {
-            const double hn = h[i] + (sr * a[cc] + ar * s[cc]);
-            h[i] = ok ? hn : h[i];
-          }
-          const double t = ::fma(h[i], x[cc], acc);
-          acc = ok ? t : acc;
-        }
-        if constexpr (PENDING) {
-#pragma unroll
-          for (int i = 0; i < kBatch; ++i)
-            hrow[int64_t(l0 + i) * NT] = h[i];
-        }
-      }
-#pragma unroll 1
-      for (int l = l0; l < Lay::L; ++l) {
-        const int col = c * Lay::L + l;
-        if (col < D) {
-          double h = hrow[int64_t(l) * NT];
-          if constexpr (PENDING) {
-            h = h + (sr * a[col] + ar * s[col]);
-            hrow[int64_t(l) * NT] = h;
-          }
-          acc = ::fma(h, x[col], acc);
-        }
-      }
-      part[c * D + row] = acc;
-    }
-  }
 };
 
 // v[row] = sum_c part[c * D + row], rows owned i = tid, tid + NT, ...
@@ -367,6 +291,224 @@ chunk_total(const double* part, int row)
   for (int c = 0; c < Lay::CH; ++c)
     t += part[c * D + row];
   return t;
+}
+
+// The inverse Hessian of a start as H = B + sum_j (s_j a_j^T + a_j s_j^T) in
+// global memory, for dimensions whose D x D matrix neither fits the registers
+// nor is worth streaming: the rank-2 pairs of the updates, B = I until the
+// list is full, then the pairs are folded into an explicit B and the list
+// restarts.  A product reads 2 k D doubles for k pairs, where a pass over an
+// explicit H reads and writes D^2 (at D = 321 they meet at k = 321 pairs); with
+// B, D^2 read and the pairs since the fold.  The list is kFirst = D / 2 pairs
+// long (at most 160) before the first fold and kLater after it: a fold costs
+// two passes over B and kLater / 2 pairs are read per product in between.
+//
+// pair_parts: partial products kept apart in LDS (the others are added in
+// rounds).
+template <int D, int NT>
+constexpr int
+pair_parts()
+{
+  return D > 512 ? 1 : (NT / kWave < 4 ? NT / kWave : 4);
+}
+template <int D, int NT>
+struct PairMatrix {
+  static constexpr bool kPairs = true;
+  static constexpr int NW = NT / kWave, EL = (D + kWave - 1) / kWave;
+  static constexpr int kFirst = D / 2 < 160 ? D / 2 : 160, kLater = 32;
+  static_assert(kLater <= kFirst, "one list for both");
+  static constexpr int kParts = pair_parts<D, NT>();
+  static constexpr int kRounds = NW / kParts;
+  static constexpr int64_t kSlabDoubles = int64_t(kFirst) * 2 * D + int64_t(D) * D;
+  double* slab = nullptr;
+  int k = 0;         // pairs in the list (the same in every thread)
+  bool base = false; // explicit B in use
+
+  ZEUS_D ZEUS_FI void set_identity()
+  {
+    k = 0;
+    base = false;
+  }
+  ZEUS_D ZEUS_FI double* explicit_b() const { return slab + int64_t(kFirst) * 2 * D; }
+
+  // part[q * D + i], q < kParts: the wavefronts' shares of (H - I) g, or of H g
+  // with an explicit B; wavefront w takes the pairs (and rows of B) w, w + NW,
+  // ..., two (four) in flight.  Ends with a barrier.
+  ZEUS_D void apply(const double* g, double* part) const
+  {
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    const int lane = threadIdx.x % kWave;
+    double gr[EL], v[EL];
+#pragma unroll
+    for (int e = 0; e < EL; ++e) {
+      const int i = lane + e * kWave;
+      gr[e] = i < D ? g[i] : 0.0;
+      v[e] = 0.0;
+    }
+    auto row = [&](const double* p, double (&r)[EL]) { // lanes past D read 0
+#pragma unroll
+      for (int e = 0; e < EL; ++e) {
+        const int i = lane + e * kWave;
+        r[e] = ((e + 1) * kWave <= D || i < D) ? p[i] : 0.0;
+      }
+    };
+    constexpr int kC = 2;
+#pragma unroll 1
+    for (int j0 = w; j0 < k; j0 += kC * NW) {
+      double s[kC][EL], a[kC][EL], c[kC], d[kC];
+#pragma unroll
+      for (int q = 0; q < kC; ++q) {
+        const int j = j0 + q * NW < k ? j0 + q * NW : j0; // past the end: not used
+        row(slab + int64_t(j) * 2 * D, s[q]);
+        row(slab + int64_t(j) * 2 * D + D, a[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < kC; ++q) {
+        c[q] = d[q] = 0.0;
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          c[q] = ::fma(a[q][e], gr[e], c[q]);
+          d[q] = ::fma(s[q][e], gr[e], d[q]);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kC; ++q) {
+        c[q] = wave_sum(c[q]);
+        d[q] = wave_sum(d[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < kC; ++q)
+        if (j0 + q * NW < k)
+#pragma unroll
+          for (int e = 0; e < EL; ++e)
+            v[e] = ::fma(s[q][e], c[q], ::fma(a[q][e], d[q], v[e]));
+    }
+    if (base) {
+      const double* B = explicit_b();
+      constexpr int kR = 4;
+#pragma unroll 1
+      for (int c0 = w; c0 < D; c0 += kR * NW) {
+        double b[kR][EL];
+#pragma unroll
+        for (int q = 0; q < kR; ++q)
+          row(B + int64_t(c0 + q * NW < D ? c0 + q * NW : c0) * D, b[q]);
+#pragma unroll
+        for (int q = 0; q < kR; ++q) {
+          const double gc = c0 + q * NW < D ? g[c0 + q * NW] : 0.0;
+#pragma unroll
+          for (int e = 0; e < EL; ++e)
+            v[e] = ::fma(b[q][e], gc, v[e]);
+        }
+      }
+    }
+#pragma unroll 1
+    for (int t = 0; t < kRounds; ++t) {
+      if (w / kParts == t) {
+        double* p = part + (w % kParts) * D;
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          const int i = lane + e * kWave;
+          if (i < D)
+            p[i] = t == 0 ? v[e] : p[i] + v[e];
+        }
+      }
+      __syncthreads();
+    }
+  }
+  // row i of H g from the parts
+  ZEUS_D ZEUS_FI double total(const double* part, const double* g, int i) const
+  {
+    double t = base ? 0.0 : g[i];
+#pragma unroll
+    for (int q = 0; q < kParts; ++q)
+      t += part[q * D + i];
+    return t;
+  }
+
+  // Appends the pair (s, a) (LDS; element i read by the thread that wrote it);
+  // the next product is behind a barrier of the caller.
+  ZEUS_D void append(const double* s, const double* a)
+  {
+    double* p = slab + int64_t(k) * 2 * D;
+    for (int i = threadIdx.x; i < D; i += NT) {
+      p[i] = s[i];
+      p[D + i] = a[i];
+    }
+    ++k;
+    if (k == (base ? kLater : kFirst))
+      fold();
+  }
+
+  // B += the pairs, kF rows at a time per wavefront.
+  ZEUS_D void fold()
+  {
+    constexpr int kF = 4;
+    __syncthreads(); // the last pair is stored
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+    const int lane = threadIdx.x % kWave;
+    double* B = explicit_b();
+#pragma unroll 1
+    for (int c0 = kF * w; c0 < D; c0 += kF * NW) {
+      double b[kF][EL];
+#pragma unroll
+      for (int q = 0; q < kF; ++q)
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          const int i = lane + e * kWave, c = c0 + q;
+          b[q][e] = !(i < D && c < D) ? 0.0 : base ? B[int64_t(c) * D + i] : i == c ? 1.0 : 0.0;
+        }
+#pragma unroll 1
+      for (int j = 0; j < k; ++j) {
+        const double* s = slab + int64_t(j) * 2 * D;
+        const double* a = s + D;
+        double sc[kF], ac[kF];
+#pragma unroll
+        for (int q = 0; q < kF; ++q) {
+          const int c = c0 + q < D ? c0 + q : D - 1;
+          sc[q] = s[c];
+          ac[q] = a[c];
+        }
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          const int i = lane + e * kWave;
+          const double si = i < D ? s[i] : 0.0, ai = i < D ? a[i] : 0.0;
+#pragma unroll
+          for (int q = 0; q < kF; ++q)
+            b[q][e] = b[q][e] + (si * ac[q] + ai * sc[q]);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kF; ++q)
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          const int i = lane + e * kWave;
+          if (i < D && c0 + q < D)
+            B[int64_t(c0 + q) * D + i] = b[q][e];
+        }
+    }
+    __syncthreads(); // before the list is overwritten and B is read
+    k = 0;
+    base = true;
+  }
+};
+
+// Storage of a start's inverse Hessian in the per-workgroup form: registers,
+// a streamed slab (up to 256 dimensions), or the pair list.
+template <int D, int NT, bool REG>
+constexpr bool kPairForm = !REG && (D > 256);
+template <int D, int NT, bool REG>
+using GroupH = std::conditional_t<kPairForm<D, NT, REG>, PairMatrix<D, NT>, DistMatrix<D, NT, REG>>;
+// its doubles of global memory per workgroup
+template <int D, int NT, bool REG>
+constexpr int64_t
+group_slab_doubles()
+{
+  if constexpr (REG)
+    return 0;
+  else if constexpr (kPairForm<D, NT, REG>)
+    return PairMatrix<D, NT>::kSlabDoubles;
+  else
+    return int64_t(RowChunk<D, NT>::kPerThread) * NT;
 }
 
 } // namespace zeus::dev

@@ -1,0 +1,73 @@
+// tanh.hpp -- hyperbolic tangent for the network objective, whose value is 32
+// of them per data point.
+//
+// tanh a = t / (t + 2), t = exp(2 a) - 1: one reduction by ln 2, the series of
+// exp to r^13 in two chains, one reciprocal with Newton steps, and the rounding
+// errors of t and of the denominator put back into the quotient.  About 60
+// instructions without a branch or a division sequence, against about 190 of
+// the library's; several neurons interleave.  Error against 113-bit: 0.88 ulp
+// at most, 0.29 ulp rms, over |x| <= 22.
+#pragma once
+
+#include "config.hpp"
+
+#include <cmath>
+
+namespace zeus::dev {
+
+ZEUS_HD ZEUS_FI double
+reciprocal(double d) // 1 / d to about an ulp, d in [2, 2^66]
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r = __builtin_amdgcn_rcp(d);
+  r = ::fma(r, ::fma(-d, r, 1.0), r);
+  return ::fma(r, ::fma(-d, r, 1.0), r);
+#else
+  return 1.0 / d;
+#endif
+}
+
+ZEUS_HD ZEUS_FI double
+tanh_unit(double x)
+{
+  const double b = ::fabs(x);
+  const double y = 2.0 * (b > 22.0 ? 22.0 : b); // tanh 22 rounds to 1; NaN stays
+  // y = k ln 2 + r, the head of ln 2 short enough for an exact product
+  const double k = ::rint(y * 1.4426950408889634074);
+  const double rh0 = ::fma(-k, 0x1.62e42fefap-1, y);
+  const double rl0 = -k * 0x1.cf79abc9e3b3ap-40;
+  const double r = rh0 + rl0;
+  const double rl = (rh0 - r) + rl0;
+  const double r2 = r * r;
+  double e = 1.0 / 479001600.0;      // 1/12!
+  double o = 1.0 / 6227020800.0;     // 1/13!
+  e = ::fma(e, r2, 1.0 / 3628800.0);
+  o = ::fma(o, r2, 1.0 / 39916800.0);
+  e = ::fma(e, r2, 1.0 / 40320.0);
+  o = ::fma(o, r2, 1.0 / 362880.0);
+  e = ::fma(e, r2, 1.0 / 720.0);
+  o = ::fma(o, r2, 1.0 / 5040.0);
+  e = ::fma(e, r2, 1.0 / 24.0);
+  o = ::fma(o, r2, 1.0 / 120.0);
+  e = ::fma(e, r2, 0.5);
+  o = ::fma(o, r2, 1.0 / 6.0);
+  // exp(r) - 1 = q + ql
+  const double rest = r2 * ::fma(o, r, e);
+  const double q = r + rest;
+  const double ql = ((r - q) + rest) + ::fma(rl, r, rl);
+  // t = 2^k (1 + q) - 1 = th + tl
+  const double s = ::ldexp(1.0, int(k));
+  const double u = s - 1.0, p = s * q;
+  const double th = u + p;
+  const double tl = ((u - th) + p) + s * ql;
+  // t / (t + 2), the denominator d + dl
+  const double d = th + 2.0;
+  const double big = th > 2.0 ? th : 2.0, small = th > 2.0 ? 2.0 : th;
+  const double dl = (small - (d - big)) + tl;
+  const double rc = reciprocal(d);
+  const double z0 = th * rc;
+  const double res = (::fma(-z0, d, th) + tl) - z0 * dl;
+  return ::copysign(::fma(res, rc, z0), x);
+}
+
+} // namespace zeus::dev

@@ -246,7 +246,7 @@ run(const F& f, double lower, double upper, std::size_t N, int MAX_ITER, int PSO
                 "occupancy");
       grid = int(std::max<int64_t>(1, std::min<int64_t>(n, int64_t(n_cu) * std::max(occ, 1))));
       if (!kHReg) {
-        stride = int64_t(RowChunk<D, NT>::kPerThread) * NT;
+        stride = group_slab_doubles<D, NT, kHReg>();
         slab = stride * grid;
       }
     } else if (D > kThreadRegMaxD) {
