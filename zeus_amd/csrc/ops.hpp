@@ -66,16 +66,17 @@ template <class F, int D>
 struct Ops {
   static constexpr bool kMfmaPso = F::id == obj::kGaussian && D >= 16;
   static constexpr bool kThreadOk = F::id != obj::kMlp && D <= 64;
-  // workgroup sizes of the group form (the MLP's cooperative evaluator puts
-  // one point per lane and one hidden-to-hidden weight per lane: 256)
+  // workgroup sizes of the group form (the MLP's cooperative evaluator has two
+  // lanes per point: 512)
   static constexpr int kNGroup = F::id == obj::kMlp ? 1 : group_nt_count(D);
-  static constexpr int nt_at(int k) { return F::id == obj::kMlp ? 256 : group_nt_at(D, k); }
+  static constexpr int nt_at(int k) { return F::id == obj::kMlp ? 512 : group_nt_at(D, k); }
   // tile form: Gaussian classes whose PSO already runs in tiles of 16
   static constexpr bool kTileOk = kMfmaPso;
   // PSO with a workgroup per particle: objectives whose one evaluation is
   // worth a workgroup (the MLP loss over its data points)
   static constexpr bool kGroupPso = F::id == obj::kMlp;
-  using PsoEval = typename dev::GroupEvalSelect<F, 256, Gradient::Adjoint>::type;
+  static constexpr int kPsoGroupThreads = 512;
+  using PsoEval = typename dev::GroupEvalSelect<F, kPsoGroupThreads, Gradient::Adjoint>::type;
   // PSO with a team of lanes per particle: the separable objectives beyond
   // four coordinates and the binned likelihood
   static constexpr int kPsoTeam = dev::pso_team_size<F, D>();
@@ -91,8 +92,8 @@ struct Ops {
     if constexpr (kMfmaPso)
       dev::pso_gaussian_mfma_kernel<D><<<nb, dev::kPsoTileThreads, 0, s>>>(a);
     else if constexpr (kGroupPso)
-      dev::pso_group_kernel<F, D, 256, kPsoPpb, PsoEval, dev::BuiltinProvider>
-        <<<nb, 256, 0, s>>>(a, {});
+      dev::pso_group_kernel<F, D, kPsoGroupThreads, kPsoPpb, PsoEval, dev::BuiltinProvider>
+        <<<nb, kPsoGroupThreads, 0, s>>>(a, {});
     else if constexpr (kPsoTeam != 0)
       dev::pso_team_kernel<F, D, kPsoTeam, dev::BuiltinProvider><<<nb, 256, 0, s>>>(a, {});
     else

@@ -18,6 +18,7 @@
 
 #include "batch.hpp"
 #include "block.hpp"
+#include "cs_product.hpp"
 #include "lane_ops.hpp"
 #include "philox.hpp"
 #include "prng.hpp"
@@ -418,157 +419,205 @@ struct GroupEvalLogLik {
 };
 
 // ---------------------------------------------------------------------------
-// MLP (1-16-16-1 tanh, least squares over m points): points spread over the
-// lanes.  Value: each lane's squared residuals, one workgroup sum.  Adjoint
-// gradient: each lane runs its point's forward and reverse sweep
-// (activations recomputed, no tape), then the sums over points are formed
-// in a fixed order: the 65 per-neuron terms (output weights and bias,
-// hidden biases, first-layer weights) by wavefront sums and a per-wavefront
-// fold, the 256 hidden-to-hidden weights as dot products over the points
-// staged in LDS (lane k*16 + j owns weight (k, j)), half a workgroup's points
-// at a time so that the staging fits two workgroups per CU.  The dual
-// gradient keeps the reference's D forward passes spread over the lanes.
+// MLP (1-16-16-1 tanh, least squares over m points), a wavefront taking 16
+// points at a time in the operand layout of the FP64 MFMA: lane l works for
+// point l % 16 and, in every layer, for the neurons 4 q + l / 16 (q < 4).  The
+// first layer's activations are then the B operand of the product with the
+// hidden weights, whose result has the second layer's neurons in the same lanes
+// and registers, and its deltas are again the B operand of the product with
+// the transposed weights.  Only the weights' own gradient d2 h1^T contracts over
+// the points and turns both 16 x 16 blocks round through LDS.  The 65
+// per-neuron gradient terms add up in registers and are summed over a row of
+// lanes once per gradient; the wavefronts' shares are added in order.
+//
+// The 32 hyperbolic tangents of a point bound it (VALU issue).  With a lane per
+// point, every weight was an LDS broadcast to every wavefront, which cost as
+// much again, and the sums over points were 65 wavefront reductions and a serial
+// product (18 us a value and 41 us a gradient).  A lane's activations of its
+// first kKeep groups stay in registers from the value to the gradient at the
+// same point.  The dual gradient keeps the reference's D forward passes spread
+// over the lanes.
 template <int NT, Gradient G>
 struct GroupEvalMlp {
   using F = obj::Mlp;
-  static constexpr int H = F::H, W2 = F::W2, W3 = F::W3;
-  static constexpr int kCols = 4 * H + 1; // w3 (16), b3, b2 (16), w1 (16), b1 (16)
-  static_assert(NT >= H * H, "one lane per hidden-to-hidden weight");
+  static constexpr bool kOneSite = true;
+  static constexpr int H = F::H, W2 = F::W2, W3 = F::W3, D = int(F::arity);
+  static constexpr int NW = NT / kWave;
+  static constexpr int kPoints = 16;            // points of a group
+  static constexpr int kKeep = 256 / (kPoints * NW); // groups kept per wavefront
+  static constexpr int Q = 4;                   // neurons per lane and layer
   GroupScratch sc;
+  struct Point { // a lane's share of its point
+    double h1[Q], h2[Q], res;
+  };
+  Point kept[kKeep];
   ZEUS_D void bind(const ProblemDesc&) {}
 
-  // forward pass of point p: hidden activations and output
-  ZEUS_D ZEUS_FI static double forward(const F& f, const double* th, int p, double (&h1)[H],
-                                       double (&h2)[H])
+  // the weights a lane needs of the forward pass
+  struct Weights {
+    double w1[Q], b1[Q], a2[Q], b2[Q], w3[Q], b3;
+    ZEUS_D ZEUS_FI explicit Weights(const double* th)
+    {
+      const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int n = 4 * q + lk;
+        w1[q] = th[2 * n];
+        b1[q] = th[2 * n + 1];
+        a2[q] = th[W2 + li * (H + 1) + n];
+        b2[q] = th[W2 + n * (H + 1) + H];
+        w3[q] = th[W3 + n];
+      }
+      b3 = th[W3 + H];
+    }
+  };
+  // forward pass of the point; all lanes of the wavefront
+  ZEUS_D ZEUS_FI static void forward(const Weights& w, double x, double y, Point& o)
   {
-    const double xp = f.P[p];
 #pragma unroll
-    for (int j = 0; j < H; ++j) {
-      double sum = 0.0;
-      sum += th[2 * j] * xp;
-      sum += th[2 * j + 1];
-      h1[j] = ::tanh(sum);
+    for (int q = 0; q < Q; ++q)
+      o.h1[q] = tanh_unit(::fma(w.w1[q], x, w.b1[q]));
+    mfma_acc_t z = {w.b2[0], w.b2[1], w.b2[2], w.b2[3]};
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      z = __builtin_amdgcn_mfma_f64_16x16x4f64(w.a2[q], o.h1[q], z, 0, 0, 0);
+    double out = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      o.h2[q] = tanh_unit(z[q]);
+      out = ::fma(o.h2[q], w.w3[q], out);
     }
-#pragma unroll 4
-    for (int k = 0; k < H; ++k) {
-      const double* w = th + W2 + k * (H + 1);
-      double sum = 0.0;
+    o.res = (xor_sum<32>(xor_sum<16>(out)) + w.b3) - y;
+  }
+  // fn(group's index in the wavefront, its point (any valid one past the end),
+  // whether it exists) over the wavefront's groups
+  template <class Fn>
+  ZEUS_D ZEUS_FI static void groups(const F& f, Fn&& fn)
+  {
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
 #pragma unroll
-      for (int j = 0; j < H; ++j)
-        sum += h1[j] * w[j];
-      sum += w[H];
-      h2[k] = ::tanh(sum);
+    for (int j = 0; j < kKeep; ++j) {
+      const int p = (w + j * NW) * kPoints + (int(threadIdx.x) & 15);
+      if ((w + j * NW) * kPoints < f.m)
+        fn(j, p < f.m ? p : f.m - 1, p < f.m);
     }
-    double sum = 0.0;
-#pragma unroll
-    for (int k = 0; k < H; ++k)
-      sum += h2[k] * th[W3 + k];
-    sum += th[W3 + H];
-    return sum;
+#pragma unroll 1
+    for (int j = kKeep; (w + j * NW) * kPoints < f.m; ++j) {
+      const int p = (w + j * NW) * kPoints + (int(threadIdx.x) & 15);
+      fn(j, p < f.m ? p : f.m - 1, p < f.m);
+    }
   }
 
   ZEUS_D double value(const F& f, const double* th, Block<NT>& blk)
   {
+    const Weights wt(th);
+    const bool counts = (threadIdx.x & 63) < 16; // one of a point's four lanes
     double t = 0.0;
-    for (int p = threadIdx.x; p < f.m; p += NT) {
-      double h1[H], h2[H];
-      const double dd = forward(f, th, p, h1, h2) - f.P[f.m + p];
-      t = ::fma(dd, dd, t);
-    }
+    groups(f, [&](auto j, int p, bool live) {
+      Point o;
+      forward(wt, f.P[p], f.P[f.m + p], o);
+      if (counts && live)
+        t = ::fma(o.res, o.res, t);
+      if (j < kKeep)
+        kept[j < kKeep ? j : 0] = o;
+    });
     return blk.sum1(t) / double(f.m);
   }
 
-  ZEUS_D void gradient(const F& f, const double* th, double* g, bool, Block<NT>& blk)
+  // the gradient at the point of the last value
+  ZEUS_D void gradient(const F& f, const double* th, double* g, bool, Block<NT>&)
   {
     if constexpr (G == Gradient::Dual) {
-      group_dual_gradient<F, int(F::arity), NT>(f, th, g);
+      group_dual_gradient<F, D, NT>(f, th, g);
     } else {
-      constexpr int kStage = NT / 2; // points staged at a time
-      __shared__ double h1s[kStage][H + 1]; // one point per lane, padded rows
-      __shared__ double d2s[kStage][H + 1];
-      __shared__ double colw[NT / kWave][kCols];
+      __shared__ double turn[NW][2][H][H + 1];
       const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+      const int li = lane & 15, lk = lane >> 4;
       const double scale = 2.0 / double(f.m);
-      for (int c = lane; c < kCols; c += kWave)
-        colw[w][c] = 0.0;
-      // per-neuron term c of this lane's point, summed over the wavefront
-      // and added to the wavefront's running total (chunks in order)
-      auto col_add = [&](int c, double v) {
-        const double t = wave_sum(v);
-        if (lane == 0)
-          colw[w][c] += t;
-      };
-      double gw = 0.0; // hidden-to-hidden weight (k, j) = (tid / H, tid % H)
-      for (int c0 = 0; c0 < f.m; c0 += NT) {
-        const int p = c0 + tid;
-        const bool live = p < f.m;
-        double h1[H], h2[H], d2[H];
-        double dy = 0.0;
-        if (live) {
-          dy = scale * (forward(f, th, p, h1, h2) - f.P[f.m + p]);
-        } else {
+      auto& A = turn[w][0];
+      auto& B = turn[w][1];
+      double a2t[Q], w3[Q]; // transposed hidden weights, output weights
 #pragma unroll
-          for (int j = 0; j < H; ++j)
-            h1[j] = h2[j] = 0.0;
-        }
+      for (int q = 0; q < Q; ++q) {
+        a2t[q] = th[W2 + (4 * q + lk) * (H + 1) + li];
+        w3[q] = th[W3 + 4 * q + lk];
+      }
+      mfma_acc_t acc = {0.0, 0.0, 0.0, 0.0}; // weights (4 q + lk, li)
+      double sw1[Q] = {}, sb1[Q] = {}, sb2[Q] = {}, sw3[Q] = {}, sb3 = 0.0;
+      groups(f, [&](auto j, int p, bool live) {
+        Point o;
+        const double x = f.P[p];
+        if (j < kKeep)
+          o = kept[j < kKeep ? j : 0];
+        else
+          forward(Weights(th), x, f.P[f.m + p], o);
+        const double dy = live ? scale * o.res : 0.0;
+        double d2[Q];
+        mfma_acc_t d1 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int k = 0; k < H; ++k) {
-          col_add(k, dy * h2[k]);                                  // w3
-          d2[k] = (dy * th[W3 + k]) * (1.0 - h2[k] * h2[k]);
-          col_add(H + 1 + k, d2[k]);                               // b2
+        for (int q = 0; q < Q; ++q) {
+          d2[q] = (dy * w3[q]) * ::fma(-o.h2[q], o.h2[q], 1.0);
+          sb2[q] += d2[q];
+          sw3[q] = ::fma(dy, o.h2[q], sw3[q]);
+          A[4 * q + lk][li] = d2[q];
+          B[4 * q + lk][li] = o.h1[q];
         }
-        col_add(H, dy);                                            // b3
-        const double xp = live ? f.P[p] : 0.0;
-#pragma unroll 4
-        for (int j = 0; j < H; ++j) {
-          double d1 = 0.0;
+        sb3 += dy;
 #pragma unroll
-          for (int k = 0; k < H; ++k)
-            d1 += d2[k] * th[W2 + k * (H + 1) + j];
-          const double dj = d1 * (1.0 - h1[j] * h1[j]);
-          col_add(2 * H + 1 + j, dj * xp);                         // w1
-          col_add(3 * H + 1 + j, dj);                              // b1
+        for (int q = 0; q < Q; ++q)
+          d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2t[q], d2[q], d1, 0, 0, 0);
+        team_exchange();
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[li][4 * q + lk], B[li][4 * q + lk], acc, 0,
+                                                     0, 0);
+        team_exchange();
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const double d = d1[q] * ::fma(-o.h1[q], o.h1[q], 1.0);
+          sb1[q] += d;
+          sw1[q] = ::fma(d, x, sw1[q]);
         }
-        // points c0 .. c0 + NT - 1 in two halves, in point order
+      });
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        sw1[q] = row_sum(sw1[q]);
+        sb1[q] = row_sum(sb1[q]);
+        sb2[q] = row_sum(sb2[q]);
+        sw3[q] = row_sum(sw3[q]);
+      }
+      sb3 = row_sum(sb3);
+      // the wavefronts' shares (kParts at a time), then their sum
+      constexpr int kParts = pair_parts<D, NT>();
 #pragma unroll 1
-        for (int half = 0; half < 2; ++half) {
-          if (tid / kStage == half) {
+      for (int t = 0; t < NW / kParts; ++t) {
+        if (w / kParts == t) {
+          double* part = sc.part + (w % kParts) * D;
+          auto put = [&](int i, double v) { part[i] = t == 0 ? v : part[i] + v; };
 #pragma unroll
-            for (int j = 0; j < H; ++j) {
-              h1s[tid % kStage][j] = h1[j];
-              d2s[tid % kStage][j] = d2[j];
+          for (int q = 0; q < Q; ++q) {
+            const int n = 4 * q + lk;
+            put(W2 + n * (H + 1) + li, acc[q]);
+            if (li == 0) {
+              put(2 * n, sw1[q]);
+              put(2 * n + 1, sb1[q]);
+              put(W2 + n * (H + 1) + H, sb2[q]);
+              put(W3 + n, sw3[q]);
             }
           }
-          __syncthreads();
-          if (tid < H * H) {
-            const int k = tid / H, j = tid % H;
-            const int left = f.m - c0 - half * kStage;
-            const int n = left < kStage ? (left > 0 ? left : 0) : kStage;
-            for (int q = 0; q < n; ++q)
-              gw = ::fma(d2s[q][k], h1s[q][j], gw);
-          }
-          __syncthreads();
+          if (lane == 0)
+            put(W3 + H, sb3);
         }
+        __syncthreads();
       }
-      for (int c = tid; c < kCols; c += NT) {
-        double t = 0.0;
-        for (int v = 0; v < NT / kWave; ++v)
-          t += colw[v][c];
-        if (c < H)
-          g[W3 + c] = t;
-        else if (c == H)
-          g[W3 + H] = t;
-        else if (c < 2 * H + 1)
-          g[W2 + (c - H - 1) * (H + 1) + H] = t;
-        else if (c < 3 * H + 1)
-          g[2 * (c - 2 * H - 1)] = t;
-        else
-          g[2 * (c - 3 * H - 1) + 1] = t;
+      for (int i = tid; i < D; i += NT) {
+        double t = sc.part[i];
+#pragma unroll
+        for (int v = 1; v < kParts; ++v)
+          t += sc.part[v * D + i];
+        g[i] = t;
       }
-      if (tid < H * H)
-        g[W2 + (tid / H) * (H + 1) + tid % H] = gw;
     }
-    (void)blk;
   }
 };
 
@@ -948,10 +997,9 @@ group_bfgs(const F& f, GroupVectors<D, NT, kPairForm<D, NT, HREG>>& L,
 // Wavefronts per SIMD the kernel is compiled for.  The binned likelihood (one
 // wavefront per start, bound by the issue of its power functions and by their
 // chains): 64 fits of 256 starts took 1.66 ms at four, 1.80 at three and 1.85
-// at two.  The MLP with the adjoint gradient alternates evaluation phases (no
-// memory traffic) with the streamed H pass (HBM bound), so two workgroups per
-// CU overlap one's pass with the other's evaluation; the register budget is
-// set for that.
+// at two.  The MLP with the adjoint gradient keeps 256 registers per lane (one
+// workgroup of eight wavefronts per CU): 512 starts x 24 iterations took 1.95
+// ms so, 2.34 ms at three wavefronts per SIMD and 2.45 ms at four, which spill.
 template <class F, Gradient G>
 constexpr int group_min_waves()
 {

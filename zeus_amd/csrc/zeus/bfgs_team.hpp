@@ -61,17 +61,6 @@ team_sum(double v)
   return v;
 }
 
-// LDS writes of a team read back by other lanes of the same wavefront: the
-// wavefront's LDS operations complete in order; these fences keep the
-// compiler from moving accesses across the exchange.
-ZEUS_D ZEUS_FI void
-team_exchange()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Value and adjoint gradient of a separable objective for a team; xl is the
 // team's point in LDS, lanes own i = r + TS k.
 template <class F, int D, int TS>

@@ -97,6 +97,17 @@ wave_sum_i64(int64_t v)
   return a + c;
 }
 
+// Sum over the 16 lanes of a row, the same bits in every lane of the row.
+ZEUS_D ZEUS_FI double
+row_sum(double v)
+{
+  v += dpp_f64<0xB1>(v);  // quad_perm [1,0,3,2]
+  v += dpp_f64<0x4E>(v);  // quad_perm [2,3,0,1]
+  v += dpp_f64<0x141>(v); // row_half_mirror
+  v += dpp_f64<0x140>(v); // row_mirror
+  return v;
+}
+
 // A value every lane of the wavefront holds identically, re-read from the
 // first active lane so that the compiler treats it as wave-uniform (scalar
 // registers) instead of one copy per lane.
@@ -132,6 +143,16 @@ wave_sum(double v)
          (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
+// LDS writes read back by other lanes of the same wavefront: the wavefront's LDS operations complete in order; these fences keep the
+// compiler from moving accesses across the exchange.
+ZEUS_D ZEUS_FI void
+team_exchange()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Deterministic workgroup sums of K values at a time.  Two LDS slots are
 // used alternately so that back-to-back reductions need one barrier each.
 template <int NT>
@@ -156,9 +177,7 @@ struct Block {
 #pragma unroll
       for (int k = 0; k < K; ++k)
         v[k] = 0.0 + v[k];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      team_exchange();
       return;
     }
     double* r = red + parity * (4 * kWaves);

@@ -20,6 +20,7 @@
 
 #include "binned.hpp"
 #include "dual.hpp"
+#include "tanh.hpp"
 #include "traits.hpp"
 #include "trig.hpp"
 
@@ -413,8 +414,12 @@ struct Mlp {
   template <class T, class X>
   ZEUS_HD T point_output(const X& th, double xp) const
   {
-    using ::tanh;
-    using dual::tanh;
+    auto tanh = [](const T& v) {
+      if constexpr (kIsDouble<T>)
+        return dev::tanh_unit(v);
+      else
+        return dual::tanh(v);
+    };
     int idx = 0;
     T h1[H], h2[H];
     for (int j = 0; j < H; ++j) {
@@ -482,14 +487,14 @@ struct Mlp {
       double sum = 0.0;
       sum += th[idx++] * xp;
       sum += th[idx++];
-      h1[j] = ::tanh(sum);
+      h1[j] = dev::tanh_unit(sum);
     }
     for (int k = 0; k < H; ++k) {
       double sum = 0.0;
       for (int j = 0; j < H; ++j)
         sum += h1[j] * th[idx++];
       sum += th[idx++];
-      h2[k] = ::tanh(sum);
+      h2[k] = dev::tanh_unit(sum);
     }
     double sum = 0.0;
     for (int k = 0; k < H; ++k)
