@@ -176,7 +176,7 @@ struct GroupEvalSeparable {
       const double t2 = x[i + 1] - x[i] * x[i];
       return t1 * t1 + 100.0 * t2 * t2;
     } else if constexpr (F::id == obj::kRastrigin) {
-      return x[i] * x[i] - 10.0 * F::cosine(x[i]);
+      return x[i] * x[i] - 10.0 * ::cos(2.0 * obj::kPi * x[i]);
     } else {
       return x[i] * x[i];
     }
@@ -262,7 +262,7 @@ struct GroupEvalSeparable {
             v[t] += t1 * t1 + 100.0 * t2 * t2;
         } else if constexpr (F::id == obj::kRastrigin) {
           if (i < D)
-            v[t] += xi * xi - 10.0 * F::cosine(xi);
+            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
         } else if constexpr (F::id == obj::kAckley) {
           if (i < D) {
             v[t] = ::fma(xi, xi, v[t]);
@@ -301,7 +301,7 @@ struct GroupEvalSeparable {
     } else if constexpr (F::id == obj::kRastrigin) {
       const double k = 10.0 * (2.0 * obj::kPi);
       for (int i = threadIdx.x; i < D; i += NT)
-        g[i] = 2.0 * x[i] + k * F::sine(x[i]);
+        g[i] = 2.0 * x[i] + k * ::sin(2.0 * obj::kPi * x[i]);
     } else if constexpr (F::id == obj::kAckley) {
       double v[2] = {0.0, 0.0};
       for (int i = threadIdx.x; i < D; i += NT) {

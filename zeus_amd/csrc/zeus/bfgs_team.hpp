@@ -76,7 +76,7 @@ struct TeamEval {
       const double t2 = x[i + 1] - x[i] * x[i];
       return t1 * t1 + 100.0 * t2 * t2;
     } else if constexpr (F::id == obj::kRastrigin) {
-      return x[i] * x[i] - 10.0 * F::cosine(x[i]);
+      return x[i] * x[i] - 10.0 * ::cos(2.0 * obj::kPi * x[i]);
     } else {
       return x[i] * x[i];
     }
@@ -141,7 +141,7 @@ struct TeamEval {
             v[t] += t1 * t1 + 100.0 * t2 * t2;
         } else if constexpr (F::id == obj::kRastrigin) {
           if (i < D)
-            v[t] += xi * xi - 10.0 * F::cosine(xi);
+            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
         } else if constexpr (F::id == obj::kAckley) {
           if (i < D) {
             v[t] = ::fma(xi, xi, v[t]);
@@ -198,7 +198,7 @@ struct TeamEval {
 #pragma unroll
       for (int k = 0; k < KC; ++k) {
         const int i = r + TS * k;
-        g[k] = i < D ? 2.0 * xl[i] + kk * F::sine(xl[i]) : 0.0;
+        g[k] = i < D ? 2.0 * xl[i] + kk * ::sin(2.0 * obj::kPi * xl[i]) : 0.0;
       }
     } else if constexpr (F::id == obj::kAckley) {
       double v0 = 0.0, v1 = 0.0;

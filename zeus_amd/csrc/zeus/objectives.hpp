@@ -22,7 +22,6 @@
 #include "dual.hpp"
 #include "tanh.hpp"
 #include "traits.hpp"
-#include "trig.hpp"
 
 #include <array>
 #include <cmath>
@@ -125,34 +124,15 @@ struct Rastrigin {
   const double* zeus_params() const { return nullptr; }
   long long zeus_n_params() const { return 0; }
 
-  // cos(2 pi x) and sin(2 pi x): beyond four dimensions by turns (trig.hpp),
-  // where the value and every trial of a line search are D of them; up to four
-  // the library's functions, whose cost the launches hide
-  ZEUS_HD static double cosine(double x)
-  {
-    if constexpr (D > 4)
-      return dev::cos_turns(x);
-    else
-      return ::cos(2.0 * kPi * x);
-  }
-  ZEUS_HD static double sine(double x)
-  {
-    if constexpr (D > 4)
-      return dev::sin_turns(x);
-    else
-      return ::sin(2.0 * kPi * x);
-  }
-
   template <class T, class X>
   ZEUS_HD T eval(const X& x) const
   {
+    using ::cos;
+    using dual::cos;
     T sum = T(10.0 * D);
     for (int i = 0; i < int(D); ++i) {
       const T xi = x[i];
-      if constexpr (kIsDouble<T>)
-        sum = sum + (xi * xi - 10.0 * cosine(xi));
-      else
-        sum = sum + (xi * xi - T(10.0) * dual::cos(xi * T(2.0 * kPi)));
+      sum = sum + (xi * xi - T(10.0) * cos(xi * T(2.0 * kPi)));
     }
     return sum;
   }
@@ -166,8 +146,9 @@ struct Rastrigin {
     const double k = 10.0 * (2.0 * kPi);
     double sum = 10.0 * D;
     for (int i = 0; i < int(D); ++i) {
-      sum += x[i] * x[i] - 10.0 * cosine(x[i]);
-      g[i] = 2.0 * x[i] + k * sine(x[i]);
+      const double w = 2.0 * kPi * x[i];
+      sum += x[i] * x[i] - 10.0 * ::cos(w);
+      g[i] = 2.0 * x[i] + k * ::sin(w);
     }
     return sum;
   }

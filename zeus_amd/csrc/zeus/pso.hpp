@@ -442,7 +442,7 @@ struct PsoTeamValue {
               t[0][i] = t1 * t1 + 100.0 * t2 * t2;
             }
           } else if constexpr (F::id == obj::kRastrigin) {
-            t[0][i] = x[i] * x[i] - 10.0 * F::cosine(x[i]);
+            t[0][i] = x[i] * x[i] - 10.0 * ::cos(x[i] * (2.0 * obj::kPi));
           } else if constexpr (F::id == obj::kAckley) {
             t[0][i] = x[i] * x[i];
             t[1][i] = ::cos(2.0 * obj::kPi * x[i]);
