@@ -18,14 +18,22 @@
 //
 // Method.  The reference's per-start BFGS (include/bfgs_sequential.cuh:
 // 46-221, utils.cuh:245-287, 376-426) with the same line search, update
-// skip rule, statuses and counters as the other forms.  The inverse Hessian
-// is kept as H = B + sum_j (s_j a_j^T + a_j s_j^T): the rank-2 pairs of the
-// update H' = H + s a^T + a s^T (a = (beta/2) s - rho u, u = H y), which is
-// the reference's update expanded; B = I until the pair list is full, then
-// the pairs are folded into an explicit B (global memory) and the list
-// restarts.  H g needs 2k dot products and 2k axpys instead of a pass over
-// D^2 entries.  Sums run in a fixed order (results are deterministic), but
-// in another order than the serial oracle: parity is to tolerance.
+// skip rule, statuses and counters as the other forms.  The update is
+// H' = H + s a^T + a s^T, a = (beta/2) s - rho u, u = H y (the reference's
+// update expanded), s = alpha p, and the next direction is p' = -H' g'.  For
+// an accepted step (g' is the gradient the update used, H g' = u - p) the two
+// give, with q0 = a.g' and the reciprocal r = -1 / (alpha p.g),
+//   a = (A alpha - r) p + r p',   A = r ((1 + rho y.u) / 2 + q0):
+// a lies in the span of the old and the new direction.  So the inverse Hessian
+// is kept as H = B + W M W^T, W the directions taken so far and M tridiagonal
+// (diagonal m, links l to the next vector): H g is one dot product and one
+// axpy per step, half of the reads, sums and axpys that the (s, a) pairs take.
+// A step that was not accepted, or whose 1 - rho s.g' = -rho alpha p.g is
+// small (below kSpanMin, where the formula would lose digits), appends a
+// itself.  B = I until the list is full, then the list is folded into an
+// explicit B (global memory) and restarts at the last direction.  Sums run in
+// a fixed order (results are deterministic), but in another order than the
+// serial oracle: parity is to tolerance.
 #pragma once
 
 #include "batch.hpp"
@@ -46,8 +54,8 @@ static_assert(kTileStarts % kTileWaves == 0, "whole slots per wavefront");
 template <int D>
 struct TileShape : CsShape<D> {
   static constexpr int EL = (D + kWave - 1) / kWave; // rows per lane in start logic
-  static constexpr int kHist = 32; // rank-2 pairs kept before folding into B
-  static constexpr int64_t kSlotDoubles = int64_t(kHist) * 2 * D + int64_t(D) * D;
+  static constexpr int kHist = 64; // vectors kept before folding into B
+  static constexpr int64_t kSlotDoubles = int64_t(kHist) * D + int64_t(D) * D;
 };
 
 struct TileArgs {
@@ -56,14 +64,15 @@ struct TileArgs {
   int64_t n_tiles;
   Control* ctl;
   StartOut out;
-  double* slot_mem; // per (workgroup, start slot): kHist pairs, then B (D x D)
+  double* slot_mem; // per (workgroup, start slot): kHist vectors, then B (D x D)
 };
 
 // Per-start state of a slot (LDS; read and written by its wavefront only).
 struct TileSlot {
   int64_t s;   // global start index
   int phase;   // 0 idle, 1 first point, 2 trial, 3 unconditional point
-  int trial, iter, grads, ls_evals, k;
+  int trial, iter, grads, ls_evals;
+  int k;       // vectors in the list; the last one is the current direction
   int base;    // explicit B in use
   double best, alpha, ddir;
 };
@@ -72,7 +81,8 @@ struct TileSlot {
 // segment held in registers across the rounds of a tile (kTileKeep >= the
 // longest segment; 24 fragments = 48 VGPRs per lane at D = 150).
 constexpr int kTileKeep = 64;
-constexpr int kHgChunk = 2; // rank-2 pairs read together in H g
+constexpr int kHgChunk = 3; // vectors read together in H g (2: 3 % slower; 4 spills)
+constexpr double kSpanMin = 0x1p-10;
 template <int D>
 using TileSeg = CsFullSeg<D, kTileWaves, kTileKeep>;
 
@@ -92,6 +102,7 @@ struct TileLds {
   // other, last read in the round before, is cleared
   int conv_sum[2];
   TileSlot slot[kTileStarts];
+  double2 ml[kTileStarts][S::kHist]; // M's diagonal and the link to the next vector
   ProblemDesc prob; // the tile's problem
 };
 
@@ -185,7 +196,8 @@ tile_slot_step(TileLds<D>& L, TileSlot& st, const int w, const ProblemDesc& P,
   double* G = L.g + w * D;
   double* Pd = L.p + w * D;
   double* hist = mem;
-  double* B = mem + int64_t(S::kHist) * 2 * D;
+  double* B = mem + int64_t(S::kHist) * D;
+  double2* ml = L.ml[w];
   int row[EL];
   bool ok[EL];
 #pragma unroll
@@ -267,7 +279,10 @@ tile_slot_step(TileLds<D>& L, TileSlot& st, const int w, const ProblemDesc& P,
       if (ok[e]) {
         G[row[e]] = g[e];
         Pd[row[e]] = -g[e];
+        hist[row[e]] = -g[e];
       }
+    ml[0] = double2{0.0, 0.0};
+    st.k = 1;
     st.best = f;
     st.grads = 1;
     begin_iteration();
@@ -295,7 +310,7 @@ tile_slot_step(TileLds<D>& L, TileSlot& st, const int w, const ProblemDesc& P,
   const bool acc = fnew < st.best;
   double gn[EL], v[EL];
   load_grad(gn);
-  // v = H gn, H = B + sum_j (s_j a_j^T + a_j s_j^T)
+  // v = H gn, H = B + W M W^T
   if (st.base) {
 #pragma unroll
     for (int e = 0; e < EL; ++e)
@@ -313,122 +328,98 @@ tile_slot_step(TileLds<D>& L, TileSlot& st, const int w, const ProblemDesc& P,
     for (int e = 0; e < EL; ++e)
       v[e] = gn[e];
   }
-  // pairs in chunks of kHgChunk: every load of a chunk is issued before its
-  // dot products (one memory latency per chunk; the pairs of the whole chip
-  // are read in the same rounds, mostly beyond the L2), the chunk's 2
-  // kHgChunk wavefront sums run side by side, then v accumulates in order j
+  // vectors in chunks of kHgChunk: every load of a chunk is issued before its
+  // dot products (one memory latency per chunk; the vectors of the whole chip
+  // are read in the same rounds, mostly beyond the L2) and the chunk's
+  // wavefront sums run side by side.  Vector j's coefficient is m_j d_j +
+  // l_{j-1} d_{j-1} + l_j d_{j+1}, so v takes vector j once d_{j+1} is there:
+  // the last vector of a chunk is carried into the next.
   constexpr int kC = kHgChunk;
-  // no LDS access is moved across the pair loop (the values it would keep
-  // live through the loop cost registers the chunk needs)
+  // no LDS access is moved across the loop (the values it would keep live
+  // through the loop cost registers the chunk needs)
   asm volatile("" ::: "memory");
+  {
+    double h[EL], ch = 0.0, dh = 0.0, lh = 0.0; // carried vector: coefficient, dot, link
+#pragma unroll
+    for (int e = 0; e < EL; ++e)
+      h[e] = 0.0;
+    const int k = __builtin_amdgcn_readfirstlane(st.k);
 #pragma unroll 1
-  for (int j0 = 0; j0 < st.k; j0 += kC) {
-    double sj[kC][EL], aj[kC][EL];
+    for (int j0 = 0; j0 < k; j0 += kC) {
+      double wj[kC][EL], d[kC];
 #pragma unroll
-    for (int c = 0; c < kC; ++c) {
-      // past the list's end the last pair is loaded again; its terms are not
-      // used.  Rows past D read the next vector of the slot (in bounds: the
-      // explicit B follows the list) and are zeroed after the load, so the
-      // loads are unconditional, addressed by a uniform base and the lane.
-      const int j = j0 + c < st.k ? j0 + c : st.k - 1;
-      const gdouble_ptr pj = as_global(hist) + int64_t(j) * 2 * D + lane;
-#pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        sj[c][e] = pj[e * kWave];
-        aj[c][e] = pj[D + e * kWave];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < kC; ++c)
-#pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        sj[c][e] = okr(e) ? sj[c][e] : 0.0;
-        aj[c][e] = okr(e) ? aj[c][e] : 0.0;
-      }
-    double cj[kC], dj[kC];
-#pragma unroll
-    for (int c = 0; c < kC; ++c) {
-      double t0 = 0.0, t1 = 0.0;
-#pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        t0 = ::fma(aj[c][e], gn[e], t0);
-        t1 = ::fma(sj[c][e], gn[e], t1);
-      }
-      cj[c] = t0;
-      dj[c] = t1;
-    }
-#pragma unroll
-    for (int c = 0; c < kC; ++c) {
-      cj[c] = wave_sum(cj[c]);
-      dj[c] = wave_sum(dj[c]);
-    }
-#pragma unroll
-    for (int c = 0; c < kC; ++c)
-      if (j0 + c < st.k)
+      for (int c = 0; c < kC; ++c) {
+        // past the list's end the last vector is loaded again; its terms are
+        // not used.  Rows past D read the next vector of the slot (in bounds:
+        // the explicit B follows the list) and are zeroed after the load, so
+        // the loads are unconditional, addressed by a uniform base and the lane.
+        const int j = j0 + c < k ? j0 + c : k - 1;
+        const gdouble_ptr pj = as_global(hist) + int64_t(j) * D + lane;
 #pragma unroll
         for (int e = 0; e < EL; ++e)
-          v[e] = ::fma(sj[c][e], cj[c], ::fma(aj[c][e], dj[c], v[e]));
+          wj[c][e] = pj[e * kWave];
+      }
+#pragma unroll
+      for (int c = 0; c < kC; ++c) {
+        double t = 0.0;
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          wj[c][e] = okr(e) ? wj[c][e] : 0.0;
+          t = ::fma(wj[c][e], gn[e], t);
+        }
+        d[c] = t;
+      }
+#pragma unroll
+      for (int c = 0; c < kC; ++c)
+        d[c] = wave_sum(d[c]);
+#pragma unroll
+      for (int c = 0; c < kC; ++c)
+        if (j0 + c < k) {
+          const double2 mc = ml[j0 + c];
+          const double c0 = ::fma(lh, d[c], ch);
+          ch = ::fma(mc.x, d[c], lh * dh);
+          dh = d[c];
+          lh = mc.y;
+#pragma unroll
+          for (int e = 0; e < EL; ++e) {
+            v[e] = ::fma(h[e], c0, v[e]);
+            h[e] = wj[c][e];
+          }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < EL; ++e)
+      v[e] = ::fma(h[e], ch, v[e]);
   }
   asm volatile("" ::: "memory");
-  // s = xt - x, y = gn - g, u = H y = H gn - H g = v + p; and |g'|^2 for
-  // the gradient g' after the iteration (gn if accepted, else g), summed as
-  // the norm of g' would be once it is stored
-  double s[EL];
-  double sTy, yu, gg;
+  // s = alpha p, y = gn - g, u = H y = H gn - H g = v + p; g' the gradient
+  // after the iteration (gn if accepted, else g)
+  double pv[EL], gv[EL];
+  load(Pd, pv);
+  load(G, gv);
+  double sTy, yu, gg, sg, ug;
   {
-    double t0 = 0.0, t1 = 0.0, t2 = 0.0;
+    double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0, t4 = 0.0;
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
-      const double xv = okr(e) ? X[row[e]] : 0.0;
-      const double xtv = okr(e) ? L.xt[row[e] * S::XS + w] : 0.0;
-      const double gv = okr(e) ? G[row[e]] : 0.0;
-      const double pv = okr(e) ? Pd[row[e]] : 0.0;
-      s[e] = xtv - xv;
-      const double y = gn[e] - gv;
-      t0 = ::fma(s[e], y, t0);
-      t1 = ::fma(y, v[e] + pv, t1);
-      const double ga = acc ? gn[e] : gv;
+      const double se = st.alpha * pv[e], y = gn[e] - gv[e], u = v[e] + pv[e];
+      const double ga = acc ? gn[e] : gv[e];
+      t0 = ::fma(se, y, t0);
+      t1 = ::fma(y, u, t1);
       t2 = ::fma(ga, ga, t2);
+      t3 = ::fma(se, ga, t3);
+      t4 = ::fma(u, ga, t4);
     }
     sTy = wave_sum(t0);
     yu = wave_sum(t1);
     gg = wave_sum(t2);
+    sg = wave_sum(t3);
+    ug = wave_sum(t4);
   }
   double dd = 0.0; // g'.p' (the next iteration's directional derivative), in row order
   const bool upd = !(::fabs(sTy) < kCurvatureSkip);
-  if (upd) {
-    const double rho = 1.0 / sTy;
-    const double beta = ::fma(rho * rho, yu, rho);
-    const double hb = 0.5 * beta;
-    double a[EL];
-    double q0, q1;
-    {
-      double t0 = 0.0, t1 = 0.0;
-#pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        const double pv = okr(e) ? Pd[row[e]] : 0.0;
-        a[e] = okr(e) ? ::fma(hb, s[e], -(rho * (v[e] + pv))) : 0.0;
-        const double ga = acc ? gn[e] : (okr(e) ? G[row[e]] : 0.0);
-        t0 = ::fma(a[e], ga, t0);
-        t1 = ::fma(s[e], ga, t1);
-      }
-      q0 = wave_sum(t0);
-      q1 = wave_sum(t1);
-    }
-    // p' = -H' g = -(H g + s (a.g) + a (s.g)), H g = v (accepted) or -p
-#pragma unroll
-    for (int e = 0; e < EL; ++e) {
-      const double ga = acc ? gn[e] : (okr(e) ? G[row[e]] : 0.0);
-      double pn = 0.0;
-      if (okr(e)) {
-        const double hg = acc ? v[e] : -Pd[row[e]];
-        pn = -::fma(a[e], q1, ::fma(s[e], q0, hg));
-        Pd[row[e]] = pn;
-      }
-      dd = ::fma(ga, pn, dd);
-    }
-    // append the pair; a full list is folded into B first
-    if (st.k == S::kHist) {
+  if (upd || acc) { // a new direction
+    if (st.k + 2 > S::kHist) { // fold the list into B first
 #pragma unroll 1
       for (int c = 0; c < D; ++c) {
         double bc[EL];
@@ -436,44 +427,85 @@ tile_slot_step(TileLds<D>& L, TileSlot& st, const int w, const ProblemDesc& P,
         for (int e = 0; e < EL; ++e)
           bc[e] = st.base ? (ok[e] ? B[int64_t(c) * D + row[e]] : 0.0)
                           : (row[e] == c ? 1.0 : 0.0);
+        double wp = 0.0, lp = 0.0, wc = hist[c]; // column c of the last and this vector
 #pragma unroll 1
-        for (int j = 0; j < S::kHist; ++j) {
-          const double* sj = hist + int64_t(j) * 2 * D;
-          const double* aj = sj + D;
-          const double sc = sj[c], ac = aj[c];
+        for (int j = 0; j < st.k; ++j) {
+          const double* wj = hist + int64_t(j) * D;
+          const double2 mc = ml[j];
+          const double wn = j + 1 < st.k ? wj[D + c] : 0.0;
+          const double cj = ::fma(mc.y, wn, ::fma(mc.x, wc, lp * wp));
 #pragma unroll
           for (int e = 0; e < EL; ++e)
             if (ok[e])
-              bc[e] = bc[e] + (sj[row[e]] * ac + aj[row[e]] * sc);
+              bc[e] = ::fma(wj[row[e]], cj, bc[e]);
+          wp = wc;
+          wc = wn;
+          lp = mc.y;
         }
 #pragma unroll
         for (int e = 0; e < EL; ++e)
           if (ok[e])
             B[int64_t(c) * D + row[e]] = bc[e];
       }
+#pragma unroll
+      for (int e = 0; e < EL; ++e)
+        if (okr(e))
+          hist[row[e]] = pv[e];
       st.base = 1;
-      st.k = 0;
+      st.k = 1;
     }
-    double* sk = hist + int64_t(st.k) * 2 * D;
+    // the new direction's place; without an update it replaces a direction
+    // that no link reaches
+    int k = !upd && (st.k == 1 || ml[st.k - 2].y == 0.0) ? st.k - 1 : st.k;
+    double2 mk = {0.0, 0.0}; // row st.k - 1 of M
+    if (upd) {
+      const double al = st.alpha;
+      const double rho = 1.0 / sTy;
+      const double hb = 0.5 * ::fma(rho * rho, yu, rho);
+      const double q0 = ::fma(hb, sg, -(rho * ug));
+      const double sd = al * st.ddir; // s.g
+      const bool span = acc && ::fabs(rho * sd) >= kSpanMin;
+      // p' = -H' g' = -(H g' + s (a.g') + a (s.g')), H g' = v (accepted) or -p
+      double a[EL];
+#pragma unroll
+      for (int e = 0; e < EL; ++e) {
+        const double se = al * pv[e];
+        a[e] = ::fma(hb, se, -(rho * (v[e] + pv[e])));
+        v[e] = -::fma(a[e], sg, ::fma(se, q0, acc ? v[e] : -pv[e]));
+      }
+      if (span) {
+        const double r = -1.0 / sd;
+        const double A = r * ::fma(0.5, ::fma(rho, yu, 1.0), q0);
+        mk = double2{2.0 * al * ::fma(A, al, -r), al * r};
+      } else {
+        double* wk = hist + int64_t(k) * D;
+#pragma unroll
+        for (int e = 0; e < EL; ++e)
+          if (okr(e))
+            wk[row[e]] = a[e];
+        ml[k++] = double2{0.0, 0.0};
+        mk.y = al;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < EL; ++e)
+        v[e] = -v[e];
+    }
+    ml[st.k - 1] = mk;
+    ml[k] = double2{0.0, 0.0};
+    double* wk = hist + int64_t(k) * D;
 #pragma unroll
     for (int e = 0; e < EL; ++e)
       if (okr(e)) {
-        sk[row[e]] = s[e];
-        sk[D + row[e]] = a[e];
+        Pd[row[e]] = v[e];
+        wk[row[e]] = v[e];
+        dd = ::fma(acc ? gn[e] : gv[e], v[e], dd);
       }
-    ++st.k;
-  } else if (acc) {
-#pragma unroll
-    for (int e = 0; e < EL; ++e) {
-      const double pn = okr(e) ? -v[e] : 0.0;
-      if (okr(e))
-        Pd[row[e]] = pn;
-      dd = ::fma(gn[e], pn, dd);
-    }
+    st.k = k + 1;
   } else {
 #pragma unroll
     for (int e = 0; e < EL; ++e)
-      dd = ::fma(okr(e) ? G[row[e]] : 0.0, okr(e) ? Pd[row[e]] : 0.0, dd);
+      dd = ::fma(gv[e], pv[e], dd);
   }
   if (acc) {
     st.best = fnew;
