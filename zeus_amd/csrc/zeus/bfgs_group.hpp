@@ -22,6 +22,7 @@
 #include "lane_ops.hpp"
 #include "philox.hpp"
 #include "prng.hpp"
+#include "trig.hpp"
 
 namespace zeus::dev {
 
@@ -188,7 +189,10 @@ struct GroupEvalSeparable {
   static constexpr int kTrials = 4;
   static constexpr int KC = (D + NT - 1) / NT;
   static constexpr bool kNext = F::id == obj::kRosenbrock;
+  // Rastrigin and Ackley: the lane's angles of the search are small
+  static constexpr bool kAngles = F::id == obj::kRastrigin || F::id == obj::kAckley;
   double tx[KC], tp[KC], nx[kNext ? KC : 1], np[kNext ? KC : 1];
+  bool small = !kAngles;
 
   ZEUS_D ZEUS_FI void trials_begin(const double* x, const double* p)
   {
@@ -201,6 +205,12 @@ struct GroupEvalSeparable {
         nx[k] = i < D - 1 ? x[i + 1] : 0.0;
         np[k] = i < D - 1 ? p[i + 1] : 0.0;
       }
+    }
+    if constexpr (kAngles) {
+      small = true;
+#pragma unroll
+      for (int k = 0; k < KC; ++k)
+        small = small && ::fabs(tx[k]) + ::fabs(tp[k]) < kSmallCoordinate;
     }
   }
   // One trial per lane, for dimensions whose value is a few operations: lane t
@@ -240,10 +250,10 @@ struct GroupEvalSeparable {
     }
   }
 
-  template <int K>
-  ZEUS_D ZEUS_FI void trials(double a0, double (&v)[K], Block<NT>& blk)
+  // the lane's terms of K trials
+  template <int K, bool Small, int KA>
+  ZEUS_D ZEUS_FI void trial_terms(double a0, double (&v)[K], double (&c)[KA]) const
   {
-    double c[F::id == obj::kAckley ? K : 1] = {};
 #pragma unroll
     for (int t = 0; t < K; ++t) {
       const double alpha = a0 * (1.0 / double(1 << t));
@@ -262,17 +272,23 @@ struct GroupEvalSeparable {
             v[t] += t1 * t1 + 100.0 * t2 * t2;
         } else if constexpr (F::id == obj::kRastrigin) {
           if (i < D)
-            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
+            v[t] += xi * xi - 10.0 * angle_cos<Small>(2.0 * obj::kPi * xi);
         } else if constexpr (F::id == obj::kAckley) {
           if (i < D) {
             v[t] = ::fma(xi, xi, v[t]);
-            c[t] += ::cos(2.0 * obj::kPi * xi);
+            c[t] += angle_cos<Small>(2.0 * obj::kPi * xi);
           }
         } else if (i < D) {
           v[t] += xi * xi;
         }
       }
     }
+  }
+  template <int K>
+  ZEUS_D ZEUS_FI void trials(double a0, double (&v)[K], Block<NT>& blk)
+  {
+    double c[F::id == obj::kAckley ? K : 1] = {};
+    by_angle(small, [&](auto sm) { trial_terms<K, sm()>(a0, v, c); });
     blk.template sum<K>(v);
     if constexpr (F::id == obj::kAckley)
       blk.template sum<K>(c);

@@ -29,6 +29,7 @@
 #include "lane_ops.hpp"
 #include "philox.hpp"
 #include "prng.hpp"
+#include "trig.hpp"
 
 namespace zeus::dev {
 
@@ -119,7 +120,17 @@ struct TeamEval {
   // from the lane's own coordinates x and p (and the next coordinate's, nx and
   // np, for Rosenbrock's coupling): value()'s terms and sums, no LDS.
   static constexpr bool kNext = F::id == obj::kRosenbrock;
-  template <int K>
+  // Small: every angle of the search is small (small_search)
+  static constexpr bool kAngles = F::id == obj::kRastrigin || F::id == obj::kAckley;
+  ZEUS_D ZEUS_FI static bool small_search(const double (&x)[KC], const double (&p)[KC])
+  {
+    bool s = true;
+#pragma unroll
+    for (int k = 0; k < KC; ++k)
+      s = s && ::fabs(x[k]) + ::fabs(p[k]) < kSmallCoordinate;
+    return s;
+  }
+  template <int K, bool Small>
   ZEUS_D ZEUS_FI static void trials(double a0, int r, const double (&x)[KC],
                                     const double (&p)[KC], const double (&nx)[KC],
                                     const double (&np)[KC], double (&v)[K])
@@ -141,11 +152,11 @@ struct TeamEval {
             v[t] += t1 * t1 + 100.0 * t2 * t2;
         } else if constexpr (F::id == obj::kRastrigin) {
           if (i < D)
-            v[t] += xi * xi - 10.0 * ::cos(2.0 * obj::kPi * xi);
+            v[t] += xi * xi - 10.0 * angle_cos<Small>(2.0 * obj::kPi * xi);
         } else if constexpr (F::id == obj::kAckley) {
           if (i < D) {
             v[t] = ::fma(xi, xi, v[t]);
-            c[t] += ::cos(2.0 * obj::kPi * xi);
+            c[t] += angle_cos<Small>(2.0 * obj::kPi * xi);
           }
         } else if (i < D) {
           v[t] += xi * xi;
@@ -166,8 +177,8 @@ struct TeamEval {
     }
   }
 
-  template <Gradient G>
-  ZEUS_D static void gradient(const F& f, const double* xl, int r, double (&g)[KC])
+  template <Gradient G, bool Small>
+  ZEUS_D ZEUS_FI static void gradient(const F& f, const double* xl, int r, double (&g)[KC])
   {
     if constexpr (G == Gradient::Dual) {
 #pragma unroll
@@ -198,7 +209,7 @@ struct TeamEval {
 #pragma unroll
       for (int k = 0; k < KC; ++k) {
         const int i = r + TS * k;
-        g[k] = i < D ? 2.0 * xl[i] + kk * ::sin(2.0 * obj::kPi * xl[i]) : 0.0;
+        g[k] = i < D ? 2.0 * xl[i] + kk * angle_sin<Small>(2.0 * obj::kPi * xl[i]) : 0.0;
       }
     } else if constexpr (F::id == obj::kAckley) {
       double v0 = 0.0, v1 = 0.0;
@@ -207,7 +218,7 @@ struct TeamEval {
         const int i = r + TS * k;
         if (i < D) {
           v0 = ::fma(xl[i], xl[i], v0);
-          v1 += ::cos(2.0 * obj::kPi * xl[i]);
+          v1 += angle_cos<Small>(2.0 * obj::kPi * xl[i]);
         }
       }
       v0 = team_sum<TS>(v0);
@@ -220,7 +231,7 @@ struct TeamEval {
 #pragma unroll
       for (int k = 0; k < KC; ++k) {
         const int i = r + TS * k;
-        g[k] = i < D ? q * xl[i] + c * ::sin(2.0 * obj::kPi * xl[i]) : 0.0;
+        g[k] = i < D ? q * xl[i] + c * angle_sin<Small>(2.0 * obj::kPi * xl[i]) : 0.0;
       }
     } else {
 #pragma unroll
@@ -319,7 +330,7 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
 
     stage(x, xl);
     double bestVal = E::value(xl, r);
-    E::template gradient<G>(f, xl, r, g);
+    E::template gradient<G, false>(f, xl, r, g);
 #pragma unroll
     for (int k = 0; k < KC; ++k)
       p[k] = -g[k];
@@ -360,9 +371,12 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
       // time; the point at 2^-20 is taken as it is
       double alpha = 1.0, fnew;
       bool found;
+      const bool small = !E::kAngles || E::small_search(x, p);
       {
         double v[1];
-        E::template trials<1>(1.0, r, x, p, nx, np, v);
+        by_angle(small, [&](auto sm) {
+          E::template trials<1, sm()>(1.0, r, x, p, nx, np, v);
+        });
         fnew = v[0];
         ++ls_evals;
         found = fnew <= ::fma(kArmijoC1, ddir, bestVal) && fnew < bestVal;
@@ -371,7 +385,9 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
       for (int t0 = 1; !found; t0 += kTrials) {
         double v[kTrials];
         const double a0 = alpha * 0.5;
-        E::template trials<kTrials>(a0, r, x, p, nx, np, v);
+        by_angle(small, [&](auto sm) {
+          E::template trials<kTrials, sm()>(a0, r, x, p, nx, np, v);
+        });
 #pragma unroll
         for (int t = 0; t < kTrials; ++t)
           if (!found) {
@@ -383,7 +399,7 @@ bfgs_team_kernel(ClassArgs a, Prov prov)
           }
       }
       stage_trial(alpha);
-      E::template gradient<G>(f, xl, r, gn);
+      by_angle(small, [&](auto sm) { E::template gradient<G, sm()>(f, xl, r, gn); });
       ++grads;
 
       // v = H g_new

@@ -28,6 +28,7 @@
 #include "lane_ops.hpp"
 #include "philox.hpp"
 #include "prng.hpp"
+#include "trig.hpp"
 
 namespace zeus::dev {
 
@@ -431,26 +432,33 @@ struct PsoTeamValue {
       }
       return v;
     } else {
+      bool small = true;
+      if constexpr (F::id == obj::kRastrigin || F::id == obj::kAckley)
 #pragma unroll
-      for (int k = 0; k < KC; ++k) {
-        const int i = r + TS * k;
-        if (i < D) {
-          if constexpr (F::id == obj::kRosenbrock) {
-            if (i < D - 1) {
-              const double t1 = 1.0 - x[i];
-              const double t2 = x[i + 1] - x[i] * x[i];
-              t[0][i] = t1 * t1 + 100.0 * t2 * t2;
+        for (int k = 0; k < KC; ++k)
+          small = small && (r + TS * k >= D || ::fabs(x[r + TS * k]) < kSmallCoordinate);
+      by_angle(small, [&](auto sm) {
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+          const int i = r + TS * k;
+          if (i < D) {
+            if constexpr (F::id == obj::kRosenbrock) {
+              if (i < D - 1) {
+                const double t1 = 1.0 - x[i];
+                const double t2 = x[i + 1] - x[i] * x[i];
+                t[0][i] = t1 * t1 + 100.0 * t2 * t2;
+              }
+            } else if constexpr (F::id == obj::kRastrigin) {
+              t[0][i] = x[i] * x[i] - 10.0 * angle_cos<sm()>(x[i] * (2.0 * obj::kPi));
+            } else if constexpr (F::id == obj::kAckley) {
+              t[0][i] = x[i] * x[i];
+              t[1][i] = angle_cos<sm()>(2.0 * obj::kPi * x[i]);
+            } else {
+              t[0][i] = x[i] * x[i];
             }
-          } else if constexpr (F::id == obj::kRastrigin) {
-            t[0][i] = x[i] * x[i] - 10.0 * ::cos(x[i] * (2.0 * obj::kPi));
-          } else if constexpr (F::id == obj::kAckley) {
-            t[0][i] = x[i] * x[i];
-            t[1][i] = ::cos(2.0 * obj::kPi * x[i]);
-          } else {
-            t[0][i] = x[i] * x[i];
           }
         }
-      }
+      });
       team_exchange();
       constexpr int n = F::id == obj::kRosenbrock ? D - 1 : D;
       double s = F::id == obj::kRastrigin ? 10.0 * D : 0.0;
