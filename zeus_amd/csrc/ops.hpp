@@ -3,6 +3,7 @@
 #pragma once
 
 #include "runtime.hpp"
+#include "zeus/bfgs_solo.hpp"
 
 #include <algorithm>
 
@@ -131,10 +132,18 @@ struct Ops {
   template <int NT>
   static constexpr bool kHReg = dev::RowChunk<D, NT>::kPerThread <= 50;
 
+  // A large Gaussian's workgroup of 512 threads with the adjoint gradient keeps
+  // the matrix in registers (bfgs_solo.hpp).
+  template <int NT>
+  static constexpr bool kSolo = F::id == obj::kGaussian && D > 64 && D <= 160 && NT == 512;
+
   template <int NT, Gradient G>
   static auto group_kernel()
   {
-    return &dev::bfgs_group_kernel<F, D, NT, G, kHReg<NT>, dev::BuiltinProvider>;
+    if constexpr (kSolo<NT> && G == Gradient::Adjoint)
+      return &dev::bfgs_solo_kernel<F, D, NT, dev::BuiltinProvider>;
+    else
+      return &dev::bfgs_group_kernel<F, D, NT, G, kHReg<NT>, dev::BuiltinProvider>;
   }
 
   template <int NT>
@@ -267,7 +276,11 @@ struct Ops {
   template <int NT>
   static constexpr int64_t slab_doubles()
   {
-    return dev::group_slab_doubles<D, NT, kHReg<NT>>();
+    constexpr int64_t n = dev::group_slab_doubles<D, NT, kHReg<NT>>();
+    if constexpr (kSolo<NT>)
+      return std::max(n, dev::SoloShape<D, NT>::kSlabDoubles);
+    else
+      return n;
   }
   static int64_t group_slab_per_block(int nt)
   {
