@@ -159,6 +159,16 @@ bin_pows(double b, double q, double x)
 {
   return {::pow(1.0 - x, b), ::pow(x, q)};
 }
+#if defined(__HIP_DEVICE_COMPILE__)
+__attribute__((noinline))
+#else
+inline
+#endif
+ZEUS_HD double
+pow_any(double y, double p)
+{
+  return ::pow(y, p);
+}
 
 // la = log(a); a_plain: a in [1e-30, 1e30].
 ZEUS_HD ZEUS_FI BinMean
@@ -191,10 +201,27 @@ bin_mean(double a, double b, double c, double d, double la, bool a_plain, double
 struct BinPow {
   double mean, ratio;
 };
+// y^p for p ln y = h, rounded (NaN: unknown).  Where h is known y is positive and
+// finite and so is p, and the compiler drops the library's selections for other
+// operands: 30 of its 224 instructions, the same bits.  64 fits of 256 starts, 100
+// bins: BFGS 1.66 -> 1.54 ms.
 ZEUS_HD ZEUS_FI double
-pow_or_limit(double y, double p, double h) // h = p ln y, rounded; NaN: unknown
+pow_or_limit(double y, double p, double h)
 {
-  return h > 711.0 ? __builtin_huge_val() : h < -747.0 ? 0.0 : ::pow(y, p);
+  if (h > 711.0)
+    return __builtin_huge_val();
+  if (h < -747.0)
+    return 0.0;
+  if (!(h == h))
+    return pow_any(y, p);
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_assume(!__builtin_isnan(y));
+  __builtin_assume(!__builtin_isinf(y));
+  __builtin_assume(!__builtin_isnan(p));
+  __builtin_assume(!__builtin_isinf(p));
+  __builtin_assume(y > 0.0);
+#endif
+  return ::pow(y, p);
 }
 ZEUS_HD ZEUS_FI BinPow
 bin_pow(double a, double b, double c, double d, double x, const BinLogs& t)
