@@ -58,8 +58,8 @@ def bfgs_flops(results, form):
     gradient (Cs x): 2 D^2 flops, E per iteration (line-search trials) plus
     one per start for its first point.  The explicit-H forms add one pass
     over H per iteration (v = H g, 2 D^2) and the rank-2 update (6 D^2).  The
-    tile form keeps H as rank-2 pairs: its per-iteration vector work is
-    O(k D) (k <= 32 pairs), under 2 % of the products at D = 150, and is
+    tile form keeps H as its directions: its per-iteration vector work is
+    O(k D) (k <= 64 directions), under 2 % of the products at D = 150, and is
     not counted."""
     f = 0.0
     for r in results:
@@ -179,7 +179,10 @@ def main() -> int:
     ms_opt = float(np.mean([r.ms_opt for r in adj]))
     flops = bfgs_flops(adj, form) / len(adj)
     achieved = flops / (ms_opt * 1e-3) / 1e12
-    if form == FORM_TILE:
+    if form == FORM_TILE and threads == 512:
+        kernel = f"bfgs_solo_kernel<150> ({threads} threads, one start per workgroup)"
+        layout = "single GPU, one workgroup per start, matrix in registers"
+    elif form == FORM_TILE:
         kernel = f"bfgs_tile_kernel<150> ({threads} threads, 16 starts per workgroup)"
         layout = "single GPU, tiles of 16 starts per workgroup (FP64 MFMA evaluation)"
     else:

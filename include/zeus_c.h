@@ -82,7 +82,11 @@ typedef int32_t zeus_status_t;
                               the team form; the autotuner picks          */
 #define ZEUS_FORM_TILE 3   /* one workgroup per tile of 16 starts, the
                               objective evaluated for the tile on FP64 MFMA
-                              (Gaussian with dim >= 16, adjoint gradient)  */
+                              (Gaussian with dim >= 16, adjoint gradient);
+                              the autotuner also tries a workgroup per start
+                              with the matrix in registers and reports it as
+                              this form with 512 threads (group_threads = 512
+                              with ZEUS_FORM_GROUP)                        */
 #define ZEUS_FORM_TEAM 4   /* teams of group_threads = 4, 8 or 16 lanes per
                               start, 64 / team starts per wavefront
                               (Rosenbrock, Rastrigin, Ackley, sphere with

@@ -376,6 +376,8 @@ struct Ops {
       o.bfgs_team = &bfgs_team;
       o.team_blocks_per_cu = &team_blocks_per_cu;
       o.tile_ok = kTileOk;
+      if constexpr (kSolo<512>)
+        o.solo_threads = 512;
       o.bfgs_tile = &bfgs_tile;
       o.tile_blocks_per_cu = &tile_blocks_per_cu;
       o.tile_slot_doubles = kTileOk ? dev::TileShape<D>::kSlotDoubles : 0;

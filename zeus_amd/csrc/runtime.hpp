@@ -39,6 +39,9 @@ struct ClassOps {
   int (*team_blocks_per_cu)(int gradient, int ts) = nullptr;
   // tile form (16 starts per workgroup, objective on MFMA; adjoint only)
   bool tile_ok = false;
+  // workgroup size at which a start has a tile to itself (bfgs_solo.hpp; the
+  // per-workgroup form's launch functions take it), 0: none
+  int solo_threads = 0;
   hipError_t (*bfgs_tile)(const dev::TileArgs&, int grid, hipStream_t) = nullptr;
   int (*tile_blocks_per_cu)() = nullptr;
   int64_t tile_slot_doubles = 0; // doubles of global memory per start slot

@@ -4,7 +4,8 @@
 // Restates the reference's tile form (include/bfgs_parallel.cuh:67-285) and
 // keeps its per-start semantics, but every lane works, not only lane 0:
 //   * H lives in the row-chunk layout of block.hpp, in registers when it
-//     fits and in a per-workgroup global slab otherwise;
+//     fits, in a per-workgroup global slab up to 256 dimensions and as a list
+//     of rank-2 pairs beyond (PairMatrix);
 //   * one read-modify-write pass over H per iteration: the rank-2 update of
 //     iteration k is applied lazily inside iteration k+1's product
 //     v = H' g_new, and since H is symmetric, u = H y = v + p and the next

@@ -406,8 +406,8 @@ pso_lane_kernel(PsoArgs a, Prov prov)
 // wavefronts.  A lane per coordinate puts them side by side and makes the
 // position and velocity rows coalesced accesses.  Whole PSO phase (11
 // launches) of one problem, lane form -> team form: binned likelihood (256
-// starts, 100 bins) 1.42 -> 0.12 ms, Rastrigin-20 (2048) 0.56 -> 0.08 ms,
-// Rosenbrock-50 (700) 0.55 -> 0.09 ms.
+// starts, 100 bins) 1.42 -> 0.098 ms (with bin_mean), Rastrigin-20 (2048) 0.56
+// -> 0.073 ms, Rosenbrock-50 (700) 0.55 -> 0.075 ms.
 template <class F, int D, int TS>
 struct PsoTeamValue {
   static constexpr int KC = (D + TS - 1) / TS;

@@ -515,12 +515,20 @@ launch_class(ClassPlan& c, Control* ctl_all, int gradient, hipStream_t st, int t
   return hipSuccess;
 }
 
+// The tile form with 16 starts to a tile; with fewer threads a start has its
+// tile to itself, launched as the per-workgroup form of that size.
+bool
+shared_tile(const TuneVal& v)
+{
+  return v.form == ZEUS_FORM_TILE && v.threads == dev::kTileThreads;
+}
+
 // Persistent grid of the group and tile forms: as many workgroups as can
 // be resident (at most one per start / per tile).
 int
 group_grid(const ClassPlan& c, const TuneVal& v, int gradient)
 {
-  if (v.form == ZEUS_FORM_TILE) {
+  if (shared_tile(v)) {
     const int occ = c.ops->tile_blocks_per_cu();
     const int g = int(std::min<int64_t>(c.pso_blocks, int64_t(g_ds.n_cu) * occ));
     return std::max(g, 1);
@@ -541,7 +549,7 @@ slab_doubles(const ClassPlan& c, const TuneVal& v, int gradient)
 {
   if (v.form == ZEUS_FORM_THREAD)
     return c.ops->thread_slab_per_start * c.total;
-  if (v.form == ZEUS_FORM_TILE)
+  if (shared_tile(v))
     return c.ops->tile_slot_doubles * dev::kTileStarts * group_grid(c, v, gradient);
   if (v.form == ZEUS_FORM_TEAM)
     return 0; // H in registers
@@ -557,7 +565,7 @@ launch_bfgs_cfg(ClassPlan& c, const TuneVal& v, Control* ctl_all, int gradient, 
     return hipSuccess;
   if (v.form == ZEUS_FORM_THREAD)
     return c.ops->bfgs_thread(a, gradient, st);
-  if (v.form == ZEUS_FORM_TILE) {
+  if (shared_tile(v)) {
     const dev::TileArgs ta{c.d_desc, c.d_block_problem, c.pso_blocks, ctl_all + c.ctl0, c.out,
                            c.h_slab};
     return c.ops->bfgs_tile(ta, group_grid(c, v, gradient), st);
@@ -730,6 +738,10 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
       if (keep.empty())
         keep.push_back({ZEUS_FORM_GROUP, c.ops->group_nt[c.ops->n_group - 1]});
       c.cands = keep;
+    } else if (opt.group_threads <= 0 && opt.gradient == ZEUS_GRAD_ADJOINT) {
+      for (auto& v : c.cands) // a tile of one start
+        if (v.form == ZEUS_FORM_GROUP && v.threads == c.ops->solo_threads)
+          v.form = ZEUS_FORM_TILE;
     }
     if (c.cands.size() > 1) {
       auto it = g_ds.tuned.find(c.key);
