@@ -70,3 +70,15 @@ def test_past_the_floor():
     assert (a["status"] == 0).all() and (a["iter"] == 200).all()
     # |x| at the floor is of the order 1e-7 at most (s.y < 1e-14 ends the updates)
     assert (a["fval"] >= 0).all() and (a["fval"] < 1e-12).all()
+
+
+def test_where_it_is_tried():
+    """Reported as the tile form; not tried where an early stop could end the
+    call before the later starts have run (more starts than CUs)."""
+    f = z.Gaussian(z.make_spd(42, 1, 150))
+    for n, required, may in ((64, 0, True), (64, 10, True), (4096, 100, False)):
+        r = z.run_batch([z.Problem(f, -5.0, 5.0, n, 10000, 10, required, 1e-8, 42)])[0]
+        form, threads = z.tuned_config(z.capi.OBJ_GAUSSIAN, 150)
+        assert form == z.capi.FORM_TILE
+        assert may or threads != 512
+        assert r.c.claimed >= min(required, n) and r.status == 1

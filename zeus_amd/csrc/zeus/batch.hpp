@@ -152,7 +152,7 @@ load_flag(const int32_t* p)
 }
 // Whether a problem can stop early at all: an iteration that cannot be stopped
 // does not wait for the flag (a device-scope load, close to a microsecond).
-ZEUS_D ZEUS_FI bool
+ZEUS_HD ZEUS_FI bool
 may_stop(const ProblemDesc& P)
 {
   return P.required > 0 && P.required <= P.n_starts;
