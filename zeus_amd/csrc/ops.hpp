@@ -81,6 +81,7 @@ struct Ops {
   // PSO with a team of lanes per particle: the separable objectives beyond
   // four coordinates and the binned likelihood
   static constexpr int kPsoTeam = dev::pso_team_size<F, D>();
+  static constexpr bool kPsoMany = F::id == obj::kLogLikelihood;
   static constexpr int kPsoPpb = kMfmaPso        ? dev::kPsoTile
                                  : kGroupPso     ? dev::kPsoGroupPpb
                                  : kPsoTeam != 0 ? 256 / (kPsoTeam != 0 ? kPsoTeam : 1)
@@ -95,8 +96,15 @@ struct Ops {
     else if constexpr (kGroupPso)
       dev::pso_group_kernel<F, D, kPsoGroupThreads, kPsoPpb, PsoEval, dev::BuiltinProvider>
         <<<nb, kPsoGroupThreads, 0, s>>>(a, {});
-    else if constexpr (kPsoTeam != 0)
+    else if constexpr (kPsoTeam != 0) {
+      if constexpr (kPsoMany)
+        if (a.ts == dev::kPsoManyTeam) {
+          dev::pso_team_kernel<F, D, dev::kPsoManyTeam, dev::BuiltinProvider>
+            <<<nb, 256, 0, s>>>(a, {});
+          return hipGetLastError();
+        }
       dev::pso_team_kernel<F, D, kPsoTeam, dev::BuiltinProvider><<<nb, 256, 0, s>>>(a, {});
+    }
     else
       dev::pso_lane_kernel<F, D, dev::BuiltinProvider><<<nb, 256, 0, s>>>(a, {});
     return hipGetLastError();
@@ -355,6 +363,7 @@ struct Ops {
       o.dim = D;
       o.pso_ppb = kPsoPpb;
       o.pso_team = kPsoTeam != 0;
+      o.pso_many_ts = kPsoMany ? dev::kPsoManyTeam : 0;
       o.pso = &pso;
       o.pso_final = &pso_final;
       o.thread_ok = kThreadOk;

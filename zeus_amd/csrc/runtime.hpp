@@ -19,6 +19,7 @@ struct ClassOps {
   int objective = 0;
   int dim = 0;
   int pso_ppb = 256; // particles per PSO workgroup
+  int pso_many_ts = 0;   // lanes per particle from kPsoMany particles on, 0: the same
   bool pso_team = false; // a workgroup may take pso_ppb x 2^k particles (team form)
   hipError_t (*pso)(const dev::PsoArgs&, int nblocks, hipStream_t) = nullptr;
   hipError_t (*pso_final)(const dev::PsoArgs&, int n_probs, hipStream_t) = nullptr;
@@ -53,9 +54,9 @@ struct ClassOps {
 // form takes more passes per workgroup once a problem would have more than
 // kPsoMaxBlocks workgroups.
 inline int
-pso_ppb_for(const ClassOps* ops, int64_t n_starts)
+pso_ppb_for(const ClassOps* ops, int64_t n_starts, int ts = 0)
 {
-  int ppb = ops->pso_ppb;
+  int ppb = ts > 0 ? 256 / ts : ops->pso_ppb;
   if (ops->pso_team)
     while ((n_starts + ppb - 1) / ppb > dev::kPsoMaxBlocks && ppb < (1 << 24))
       ppb *= 2;

@@ -54,6 +54,7 @@ struct PsoArgs {
   int64_t xw_stride;
   int32_t keep_rng = 0; // store the states after the last iteration too (PSO phases)
   int32_t ppb = 256;    // particles per workgroup
+  int32_t ts = 0;      // team form: lanes per particle where not pso_team_size's
 };
 
 // (value, index) order for argmin: NaN loses to any number, ties and the
@@ -494,6 +495,13 @@ pso_team_size()
   else
     return 0;
 }
+
+// The likelihood with many particles in a launch: 16 lanes each, so that a
+// wavefront's serial sums serve four particles.  11 launches of 16384 particles,
+// 100 bins: 0.476 ms with 64 lanes, 0.333 with 32, 0.292 with 16; of 256 particles
+// 0.098, 0.113 and 0.136.  The lines cross near 2800 particles.
+constexpr int kPsoManyTeam = 16;
+constexpr int64_t kPsoMany = 4096;
 
 // a.ppb = kTeams * passes particles per workgroup: one pass while a problem's
 // workgroups number no more than kPsoMaxBlocks (every workgroup folds all of

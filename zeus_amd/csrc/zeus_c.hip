@@ -367,6 +367,7 @@ struct ClassPlan {
   int64_t total = 0;
   int pso_blocks = 0;
   int ppb = 256; // particles per PSO workgroup
+  int pso_ts = 0; // PsoArgs::ts
   int max_pso_iter = -1;
   TuneVal cfg{};
   std::vector<TuneVal> cands; // > 1 entry: time them and keep the fastest
@@ -479,7 +480,7 @@ pso_args(const ClassPlan& c, Control* ctl)
                  c.part_val, c.part_idx,
                  c.part_x,   c.gstate,
                  c.d_block_problem, c.xw,
-                 c.total * c.ops->dim, c.keep_rng, c.ppb};
+                 c.total * c.ops->dim, c.keep_rng, c.ppb, c.pso_ts};
 }
 
 // Objective preparation and PSO iterations t0 .. max_pso_iter of a class.
@@ -684,11 +685,14 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
   for (auto& c : classes) {
     c.ctl0 = ctl_total;
     ctl_total += int(c.probs.size());
-    int64_t s0 = 0, n_max = 0;
+    int64_t s0 = 0, n_max = 0, n_all = 0;
     int b0 = 0;
-    for (int pi : c.probs)
+    for (int pi : c.probs) {
       n_max = std::max(n_max, probs[pi].n_starts);
-    c.ppb = rt::pso_ppb_for(c.ops, n_max);
+      n_all += probs[pi].n_starts;
+    }
+    c.pso_ts = n_all >= dev::kPsoMany ? c.ops->pso_many_ts : 0;
+    c.ppb = rt::pso_ppb_for(c.ops, n_max, c.pso_ts);
     for (int pi : c.probs) {
       const zeus_problem& p = probs[pi];
       ProblemDesc d{};
