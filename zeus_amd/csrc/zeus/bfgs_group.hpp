@@ -41,7 +41,7 @@ template <class F, int D, int NT, Gradient G>
 struct GroupEvalLane {
   GroupScratch sc;
   int par = 0;
-  ZEUS_D void bind(const ProblemDesc&) {}
+  ZEUS_D void bind(const F&, const ProblemDesc&) {}
   ZEUS_D double value(const F& f, const double* x, Block<NT>&)
   {
     double* b = sc.scalar + par;
@@ -86,7 +86,7 @@ struct GroupEvalGaussian {
   const double* Cs = nullptr;
   GroupScratch sc;
 
-  ZEUS_D void bind(const ProblemDesc& P)
+  ZEUS_D void bind(const F&, const ProblemDesc& P)
   {
     Cs = P.aux;
     if constexpr (kReg)
@@ -150,7 +150,7 @@ struct GroupEvalGaussian {
 template <class F, int D, int NT, Gradient G>
 struct GroupEvalSeparable {
   GroupScratch sc;
-  ZEUS_D void bind(const ProblemDesc&) {}
+  ZEUS_D void bind(const F&, const ProblemDesc&) {}
 
   ZEUS_D double value(const F&, const double* x, Block<NT>& blk)
   {
@@ -392,11 +392,11 @@ struct GroupEvalLogLik {
   GroupScratch sc;
   Lds* L;
 
-  ZEUS_D void bind(const ProblemDesc& P)
+  // the bins are the functor's: a caller's own functor (zeus.hpp) has none in P
+  ZEUS_D void bind(const F& f, const ProblemDesc&)
   {
     __shared__ Lds lds;
     L = &lds;
-    const F f{P.params, int(P.n_params / 3), P.aux};
     for (int i = threadIdx.x; i < f.n && i < kKeep; i += NT) {
       const F::Bin b = f.bin(i);
       const double v[kFields] = {b.x, b.k, b.lgk, b.t.lx, b.t.l1};
@@ -500,7 +500,7 @@ struct GroupEvalMlp {
     double h1[Q], h2[Q], res;
   };
   Point kept[kKeep];
-  ZEUS_D void bind(const ProblemDesc&) {}
+  ZEUS_D void bind(const F&, const ProblemDesc&) {}
 
   // the weights a lane needs of the forward pass
   struct Weights {
@@ -1113,11 +1113,11 @@ bfgs_group_kernel(ClassArgs a, Prov prov)
   for (int64_t s = blockIdx.x; s < a.total_starts; s += gridDim.x) {
     const int pi = find_problem(a.probs, a.n_probs, s);
     const ProblemDesc P = a.probs[pi];
+    decltype(auto) f = prov.template get<F>(P);
     if (pi != bound) {
-      ev.bind(P);
+      ev.bind(f, P);
       bound = pi;
     }
-    decltype(auto) f = prov.template get<F>(P);
     group_bfgs<F, D, NT, G, HREG>(f, L, H, ev, blk, P, a.ctl + pi, s, a.starts, a.out);
   }
 }

@@ -622,8 +622,8 @@ pso_group_kernel(PsoArgs a, Prov prov)
   Block<NT> blk{red};
   Eval ev;
   ev.sc = GroupScratch{nullptr, stash, scalar};
-  ev.bind(P);
   decltype(auto) f = prov.template get<F>(P);
+  ev.bind(f, P);
   const int tid = threadIdx.x;
   double bv = __builtin_nan("");
   int64_t bi = int64_t(1) << 62;
