@@ -1052,6 +1052,9 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
       key.push_back(uint64_t(reinterpret_cast<uintptr_t>(c.ops)));
       key.push_back(uint64_t(c.total));
       key.push_back(uint64_t(c.pso_blocks));
+      // launch arguments chosen per call: neither follows from the counts
+      key.push_back(uint64_t(c.ppb));
+      key.push_back(uint64_t(c.pso_ts));
       key.push_back(uint64_t(int64_t(c.max_pso_iter)));
       key.push_back(uint64_t(c.probs.size()));
       key.push_back(uint64_t(c.cfg.form) << 32 | uint32_t(c.cfg.threads));
