@@ -105,6 +105,7 @@ struct DeviceState {
   size_t arena_bytes = 0;
   void* pinned = nullptr; // host mirror of the arena's upload/download regions
   size_t pinned_bytes = 0;
+  int pinned_idle = 0; // calls in a row that needed little of it
   std::map<TuneKey, TuneVal> tuned; // autotuner results (only tuned choices)
   std::map<std::tuple<int, int, int>, TuneVal> last; // last shape used per class and gradient
   struct Graph {
@@ -208,13 +209,22 @@ arena_reserve(size_t bytes)
   return ZEUS_OK;
 }
 
-// Grow-only pinned host buffer (a fresh allocation: pinned memory is
-// allocated, never registered after the fact).
+// Pinned host buffer (a fresh allocation: pinned memory is allocated, never
+// registered after the fact).  It grows as needed and holds the staged per-start
+// outputs too (bounded, zeus_run_batch); a large one is given back once
+// kPinnedIdle calls in a row had no use for a quarter of it.
+constexpr size_t kPinnedKept = size_t(4) << 20;
+constexpr int kPinnedIdle = 64;
 zeus_status_t
 pinned_reserve(size_t bytes)
 {
-  if (bytes <= g_ds.pinned_bytes)
-    return ZEUS_OK;
+  if (bytes <= g_ds.pinned_bytes) {
+    const bool idle = g_ds.pinned_bytes > kPinnedKept && bytes < g_ds.pinned_bytes / 4;
+    g_ds.pinned_idle = idle ? g_ds.pinned_idle + 1 : 0;
+    if (g_ds.pinned_idle < kPinnedIdle)
+      return ZEUS_OK;
+  }
+  g_ds.pinned_idle = 0;
   if (g_ds.pinned) {
     (void)hipHostFree(g_ds.pinned);
     g_ds.pinned = nullptr;
