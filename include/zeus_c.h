@@ -85,8 +85,9 @@ typedef int32_t zeus_status_t;
                               (Gaussian with dim >= 16, adjoint gradient);
                               the autotuner also tries a workgroup per start
                               with the matrix in registers and reports it as
-                              this form with 512 threads (group_threads = 512
-                              with ZEUS_FORM_GROUP)                        */
+                              this form with 512 threads, under which it can
+                              be asked for (group_threads = 512; also with
+                              ZEUS_FORM_GROUP)                             */
 #define ZEUS_FORM_TEAM 4   /* teams of group_threads = 4, 8 or 16 lanes per
                               start, 64 / team starts per wavefront
                               (Rosenbrock, Rastrigin, Ackley, sphere with
@@ -146,7 +147,9 @@ typedef struct zeus_problem {
 typedef struct zeus_options {
   int32_t gradient;      /* ZEUS_GRAD_*                                    */
   int32_t form;          /* ZEUS_FORM_*                                    */
-  int32_t group_threads; /* workgroup size of the group form (0 = tuned)   */
+  int32_t group_threads; /* workgroup size of the group form (0 = tuned)
+                            and team size of the team form; 512 with the
+                            tile form: its form of one start per workgroup */
   int32_t nzerosteps;    /* accepted for API parity; inert (the line search
                             never returns a zero step)                     */
   int32_t use_graph;     /* capture the launch sequence once per batch

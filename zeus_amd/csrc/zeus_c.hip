@@ -337,8 +337,11 @@ candidates(const ClassOps* ops, const zeus_options& opt)
 {
   std::vector<TuneVal> v;
   const bool tile_ok = ops->tile_ok && opt.gradient == ZEUS_GRAD_ADJOINT;
-  if (opt.form == ZEUS_FORM_TILE && tile_ok)
-    return {{ZEUS_FORM_TILE, dev::kTileThreads}};
+  if (opt.form == ZEUS_FORM_TILE && tile_ok) {
+    // a tile of one start (shared_tile) has the per-workgroup form's size
+    const bool solo = ops->solo_threads > 0 && opt.group_threads == ops->solo_threads;
+    return {{ZEUS_FORM_TILE, solo ? ops->solo_threads : dev::kTileThreads}};
+  }
   const bool want_thread = opt.form == ZEUS_FORM_THREAD || opt.form == ZEUS_FORM_AUTO;
   const bool want_group =
     opt.form == ZEUS_FORM_GROUP || opt.form == ZEUS_FORM_AUTO || !ops->thread_ok;
@@ -787,10 +790,17 @@ zeus_run_batch(const zeus_problem* probs, int32_t n_probs, const zeus_options* o
     }
     if (c.cands.size() > 1) {
       auto it = g_ds.tuned.find(c.key);
-      if (it != g_ds.tuned.end())
+      if (it != g_ds.tuned.end()) {
+        TuneVal t = it->second;
+        // a recorded call runs a tile of one start under its other name
+        if (c.traced && t.form == ZEUS_FORM_TILE && !shared_tile(t))
+          t.form = ZEUS_FORM_GROUP;
         for (const auto& v : c.cands)
-          if (v.form == it->second.form && v.threads == it->second.threads)
+          if (v.form == t.form && v.threads == t.threads) {
             c.cands = {v};
+            break;
+          }
+      }
     }
     if (c.traced && c.cands.size() > 1)
       c.cands.resize(1);
