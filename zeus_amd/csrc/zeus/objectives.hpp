@@ -318,16 +318,31 @@ struct LogLikelihood {
     return -(v.k * m.log_mean - m.mean - v.lgk);
   }
 
-  // one bin's contribution to the log-likelihood in dual numbers
+  // one bin's contribution to the log-likelihood in the numbers T_ (dual, or any
+  // with these functions)
+  template <class T_, class X>
+  ZEUS_HD T_ bin_log_p(const X& th, int i) const
+  {
+    using ::log;
+    using ::pow;
+    using dual::log;
+    using dual::pow;
+    const T_ a = th[0], b = th[1], c = th[2], d = th[3];
+    const T_ x = T_(P[i]);
+    const T_ k = T_(P[n + i]);
+    const T_ mean = a * pow(T_(1.0) - x, b) / pow(x, c + d * log(x));
+    return k * log(mean) - mean - T_(P[2 * n + i]);
+  }
   template <class X>
   ZEUS_HD DualNumber bin_dual(const X& th, int i) const
   {
-    const DualNumber a = th[0], b = th[1], c = th[2], d = th[3];
-    const DualNumber x = DualNumber(P[i]);
-    const DualNumber k = DualNumber(P[n + i]);
-    const DualNumber mean =
-      a * dual::pow(DualNumber(1.0) - x, b) / dual::pow(x, c + d * dual::log(x));
-    return k * dual::log(mean) - mean - DualNumber(P[2 * n + i]);
+    return bin_log_p<DualNumber>(th, i);
+  }
+  // one bin's value
+  ZEUS_HD double bin_value(const double* th, int i) const
+  {
+    const Bin e = bin(i);
+    return pow_term(e, dev::bin_pow(th[0], th[1], th[2], th[3], e.x, e.t));
   }
   // one bin's value and gradient terms from its mean by power functions
   ZEUS_HD static double pow_term(const Bin& e, const dev::BinPow& m)
@@ -355,7 +370,7 @@ struct LogLikelihood {
       }
     } else {
       for (int i = 0; i < n; ++i)
-        nll -= bin_dual(th, i);
+        nll -= bin_log_p<T_>(th, i);
     }
     return nll;
   }
@@ -395,11 +410,13 @@ struct Mlp {
   template <class T, class X>
   ZEUS_HD T point_output(const X& th, double xp) const
   {
-    auto tanh = [](const T& v) {
+    auto act = [](const T& v) -> T {
+      using ::tanh;
+      using dual::tanh;
       if constexpr (kIsDouble<T>)
         return dev::tanh_unit(v);
       else
-        return dual::tanh(v);
+        return tanh(v);
     };
     int idx = 0;
     T h1[H], h2[H];
@@ -409,7 +426,7 @@ struct Mlp {
       ++idx;
       sum += th[idx];
       ++idx;
-      h1[j] = tanh(sum);
+      h1[j] = act(sum);
     }
     for (int k = 0; k < H; ++k) {
       T sum = T(0.0);
@@ -419,7 +436,7 @@ struct Mlp {
       }
       sum += th[idx];
       ++idx;
-      h2[k] = tanh(sum);
+      h2[k] = act(sum);
     }
     T sum = T(0.0);
     for (int k = 0; k < H; ++k) {
