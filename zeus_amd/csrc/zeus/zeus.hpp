@@ -49,6 +49,7 @@
 #include <stdexcept>
 #include <string>
 #include <string_view>
+#include <type_traits>
 #include <vector>
 
 namespace zeus {
@@ -207,6 +208,14 @@ run(const F& f, double lower, double upper, std::size_t N, int MAX_ITER, int PSO
                        tr->alpha ? t_alpha.data() : nullptr, int32_t(t_steps),
                        int32_t(t_starts)};
     }
+    // obj::Gaussian: its cooperative evaluator reads the symmetric matrix
+    constexpr bool kGaussian = std::is_same_v<F, obj::Gaussian<std::size_t(D)>>;
+    HipBuffer<double> aux(kGaussian && parallel ? gaussian_aux_doubles(D) : 0);
+    if constexpr (kGaussian) {
+      P.params = f.C;
+      P.n_params = int64_t(D) * D;
+      P.aux = aux.data();
+    }
     HipBuffer<ProblemDesc> dP(1);
     abi_check(zeus_memcpy_h2d(dP.data(), &P, sizeof(P)), "upload");
     HipBuffer<Control> ctl(1);
@@ -263,6 +272,9 @@ run(const F& f, double lower, double upper, std::size_t N, int MAX_ITER, int PSO
     hip_check(hipEventCreateWithFlags(&e1, hipEventDisableSystemFence), "event");
     init_controls_kernel<<<1, 256, 0, s>>>(ctl.data(), 1, gbx.data(), D);
     hip_check(hipEventRecord(ep, s), "event");
+    if (kGaussian && parallel)
+      symmetrize_kernel<<<int((gaussian_aux_doubles(D) + 255) / 256), 256, 0, s>>>(
+        dP.data(), 0, aux.data(), aux.data() + int64_t(D) * D, D);
     if (pso) {
       PsoArgs pa{dP.data(),       1,           0,           nblk,           ctl.data(),
                  X.data(),        V.data(),    pbx.data(),  pbv.data(),     gbx.data(),
