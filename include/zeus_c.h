@@ -236,7 +236,8 @@ zeus_status_t zeus_pso_run(const zeus_problem* prob, double* pbest_x,
    the caller's outputs (positions, velocities, per-workgroup partials, the
    Gaussian's prepared matrix, XORWOW states, the control block) lives in a
    fixed 32 MiB device array of the library, one per GPU, held until the
-   process ends.  A problem whose buffers exceed it returns ZEUS_E_SCRATCH
+   process ends (the likelihood's table of logarithms, for up to 16384 bins, in
+   a second one of 512 KiB that zeus_eval uses too).  A problem whose buffers exceed it returns ZEUS_E_SCRATCH
    (up to about 0.8e6 start-coordinates with XORWOW draws and 2e6 with
    PHILOX / SOBOL: 4096 starts x 150 dimensions fit under every generator).  The array keeps the last call's
    contents; calls are serialized by the library and each returns after its
@@ -280,7 +281,8 @@ zeus_status_t zeus_bfgs_update(double* H, const double* s, const double* y,
                                int64_t batch, int32_t n, void* stream);
 
 /* Objective values (and gradients when grad != NULL) at n points (device
-   arrays, x: n x dim), lane per point; gradient ZEUS_GRAD_*. */
+   arrays, x: n x dim), a lane per point (the likelihood: 16 lanes, its sum over
+   the bins in another order); gradient ZEUS_GRAD_*. */
 zeus_status_t zeus_eval(const zeus_problem* prob, const double* x, int64_t n,
                         double* f, double* grad, int32_t gradient,
                         void* stream);

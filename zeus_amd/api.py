@@ -528,7 +528,7 @@ def bfgs_update(H, s, y) -> np.ndarray:
 
 
 def evaluate(f: Objective, X, gradient: str | None = None):
-    """Values (and gradients) at the rows of X, one lane per point."""
+    """Values (and gradients) at the rows of X (zeus_eval)."""
     X = np.ascontiguousarray(X, np.float64).reshape(-1, f.dim)
     n = X.shape[0]
     addr, nparam = f.device_params()

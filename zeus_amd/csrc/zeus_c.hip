@@ -1469,7 +1469,7 @@ pso_phase(const zeus_problem* prob, int t0, int t1, double* X, double* V, double
 // ---- fixed device scratch of the allocation-free PSO entry point ----------
 // One array per GPU the library runs on, held until the process ends.  Its
 // name is a host-side stand-in: host code uses only the address that
-// hipGetSymbolAddress returns for the current device (scratch_base).
+// hipGetSymbolAddress returns for the current device (fixed_arrays).
 constexpr size_t kScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
