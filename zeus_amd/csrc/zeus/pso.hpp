@@ -505,7 +505,8 @@ pso_team_size()
 // 4096 0.181 against 0.154, 16384 0.500 against 0.288 (32 lanes 0.333); 200 bins,
 // 2800 0.149 against 0.215, 4096 0.226 against 0.215; 50 bins, 2800 0.106 against
 // 0.121, 4096 0.155 against 0.120.  The lines cross between 2800 and 4096 (10 bins:
-// 16 lanes are level or ahead from 512 on, by 0.015 at 2800).
+// 16 lanes are level or ahead from 512 on, by 0.015 at 2800).  zeus_run_batch
+// takes them; the PSO entry points keep 64 lanes, with the same bits.
 constexpr int kPsoManyTeam = 16;
 constexpr int64_t kPsoMany = 4096;
 
