@@ -557,7 +557,7 @@ group_grid(const ClassPlan& c, const TuneVal& v, int gradient)
   }
   if (v.form == ZEUS_FORM_TEAM) {
     const int64_t teams = dev::kTeamThreads / v.threads;
-    const int64_t most = c.beside ? int64_t(1) << 24
+    const int64_t most = c.beside ? int64_t(1) << 22 // (a launch has below 2^32 threads)
                                   : int64_t(g_ds.n_cu) *
                                       c.ops->team_blocks_per_cu(gradient, v.threads);
     const int g = int(std::min<int64_t>((c.total + teams - 1) / teams, most));
